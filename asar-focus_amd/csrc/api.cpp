@@ -206,6 +206,41 @@ float2* get_twiddles(asarf_ctx* c, int n, int* status) {
     return d;
 }
 
+const float4* get_rc_twiddles(asarf_ctx* c, int n, int* status) {
+    auto it = c->rc_tables.find(n);
+    if (it != c->rc_tables.end()) return it->second;
+    int radix[kMaxPasses];
+    const int np = rc_block_radices(n, radix);
+    if (np == 0) {
+        *status = set_error(ASARF_EUNSUPPORTED, "no block range compression of length %d", n);
+        return nullptr;
+    }
+    std::vector<float2> h;
+    int ns = radix[0];
+    for (int p = 1; p < np; ++p) {
+        const int r = radix[p];
+        for (int q = 0; q < r; q += 2)  // pairs of exponents
+            for (int k = 0; k < ns; ++k)
+                for (int e = q; e < q + 2; ++e) {
+                    const double a = -2.0 * M_PI * (double)((long)e * k) / (double)((long)ns * r);
+                    h.push_back(make_float2((float)std::cos(a), (float)std::sin(a)));
+                }
+        ns *= r;
+    }
+    float4* d = nullptr;
+    if (hipMalloc(&d, sizeof(float2) * h.size()) != hipSuccess) {
+        *status = set_error(ASARF_ENOMEM, "range compression twiddles of length %d", n);
+        return nullptr;
+    }
+    if (hipMemcpy(d, h.data(), sizeof(float2) * h.size(), hipMemcpyHostToDevice) != hipSuccess) {
+        (void)hipFree(d);
+        *status = set_error(ASARF_EHIP, "range compression twiddles of length %d: upload", n);
+        return nullptr;
+    }
+    c->rc_tables[n] = d;
+    return d;
+}
+
 const FftPlanHost* get_plan(asarf_ctx* c, int n, int lanes, int* status) {
     if (lanes == kRowThreads) {
         auto t = c->tuned_rows.find(n);
@@ -306,6 +341,7 @@ extern "C" int asarf_ctx_destroy(asarf_ctx* c) {
         (void)hipSetDevice(c->device);
         (void)hipStreamSynchronize(c->stream);
         for (auto& kv : c->tw_tables) (void)hipFree(kv.second);
+        for (auto& kv : c->rc_tables) (void)hipFree(kv.second);
         if (c->d_scratch) (void)hipFree(c->d_scratch);
         if (c->h_pinned) (void)hipHostFree(c->h_pinned);
         if (c->own_stream && c->stream) (void)hipStreamDestroy(c->stream);
@@ -563,6 +599,13 @@ extern "C" int asarf_doppler_centroid(asarf_ctx* c, const asarf_image* img, doub
     return clear_error();
 }
 
+namespace asarf {
+bool chirp_tail_zero(const float* chirp_iq, int nc, int n) {
+    for (long i = 2L * nc; i < 2L * n; ++i)
+        if (chirp_iq[i] != 0.0f) return false;
+    return true;
+}
+
 // conj(FFT(chirp)) / n into d_h (device, n complex). Uses d_h as the transform buffer.
 static int chirp_spectrum(asarf_ctx* c, const float* chirp_iq, int n, float2* d_h) {
     int st = ASARF_OK;
@@ -585,6 +628,14 @@ static int chirp_spectrum(asarf_ctx* c, const float* chirp_iq, int n, float2* d_
     return ASARF_OK;
 }
 
+int rc_block_spectrum(asarf_ctx* c, const float* chirp_iq, int nc, int n, float2* d_h) {
+    HIP_CHECK(hipMemcpyAsync(d_h + n, chirp_iq, sizeof(float2) * (size_t)nc, hipMemcpyHostToDevice, c->stream));
+    HIP_CHECK(launch_rc_block_spectrum(d_h + n, nc, n, d_h, c->stream));
+    HIP_CHECK(hipStreamSynchronize(c->stream));  // the caller's chirp outlives the copy
+    return ASARF_OK;
+}
+}  // namespace asarf
+
 extern "C" int asarf_range_compression(asarf_ctx* c, asarf_image* img, const float* chirp_iq, int n_chirp, int nc,
                                        asarf_workspace* ws) {
     if (!c || !chirp_iq) return set_error(ASARF_EINVAL, "asarf_range_compression: null argument");
@@ -596,25 +647,39 @@ extern "C" int asarf_range_compression(asarf_ctx* c, asarf_image* img, const flo
         return set_error(ASARF_EINVAL, "asarf_range_compression: chirp samples %d vs range size %d", nc, img->x_size);
     ST_CHECK(ctx_init(c));
     int st = ASARF_OK;
-    const FftPlanHost* p = get_plan(c, n_chirp, kRowThreads, &st);
+    const FftPlanHost* p = get_plan(c, n_chirp, kRowThreads, &st);  // lengths without a transform stay refused
     if (!p) return st;
-    void* scratch = nullptr;
-    ST_CHECK(ctx_scratch(c, sizeof(float2) * (size_t)n_chirp, &scratch));
-    float2* d_h = static_cast<float2*>(scratch);
-    ST_CHECK(chirp_spectrum(c, chirp_iq, n_chirp, d_h));
     RcArgs a{};
     a.in = img->data;
     a.in_stride = img->x_stride;
-    a.nr_in = img->x_stride;
     a.out = static_cast<float2*>(img->data);
     a.out_stride = img->x_stride;
     a.rows = img->y_size;
     a.nrv = img->x_size - nc;
     a.zero_to = img->x_stride;
     a.coef = nullptr;
+    // The lines are compressed in place, so the block kernel takes a whole line: the shortest compiled length that
+    // holds the logical samples, when the chirp ends within its nc samples; else the transform of the padded line.
+    RcBlock rb{};
+    const bool block = chirp_tail_zero(chirp_iq, nc, n_chirp) && rc_block_choose(img->x_size, nc, true, &rb);
+    const int n = block ? rb.n : n_chirp;
+    void* scratch = nullptr;
+    ST_CHECK(ctx_scratch(c, sizeof(float2) * (size_t)n * 2, &scratch));
+    float2* d_h = static_cast<float2*>(scratch);
+    ST_CHECK(block ? rc_block_spectrum(c, chirp_iq, nc, n, d_h) : chirp_spectrum(c, chirp_iq, n_chirp, d_h));
     a.hconj = d_h;
-    a.plan = p->dev();
-    HIP_CHECK(launch_range_compress(a, RAW_CF32, c->stream));
+    if (block) {
+        a.nr_in = img->x_size;
+        a.blocks = rb.blocks;
+        a.block_step = rb.step;
+        a.rc_tw = get_rc_twiddles(c, n, &st);
+        if (!a.rc_tw) return st;
+        HIP_CHECK(launch_rc_block(a, RAW_CF32, n, c->stream));
+    } else {
+        a.nr_in = img->x_stride;
+        a.plan = p->dev();
+        HIP_CHECK(launch_range_compress(a, RAW_CF32, c->stream));
+    }
     img->x_size = a.nrv;
     return clear_error();
 }

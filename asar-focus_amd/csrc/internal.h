@@ -58,6 +58,7 @@ struct asarf_ctx {
     // plan caches keyed by (length, lanes per transform)
     std::map<std::pair<int, int>, std::unique_ptr<asarf::FftPlanHost>> plans;
     std::map<int, float2*> tw_tables;
+    std::map<int, float4*> rc_tables;  // per block length: the twiddles of the block range compression's passes
     // grow-only scratch
     void* d_scratch = nullptr;
     size_t scratch_bytes = 0;
@@ -81,6 +82,12 @@ int ctx_scratch(asarf_ctx* ctx, size_t bytes, void** out);
 int ctx_pinned(asarf_ctx* ctx, size_t bytes, void** out);
 const FftPlanHost* get_plan(asarf_ctx* ctx, int n, int lanes, int* status);
 float2* get_twiddles(asarf_ctx* ctx, int n, int* status);
+// Block range compression (rc_block.h): the pass twiddles of block length n.
+const float4* get_rc_twiddles(asarf_ctx* ctx, int n, int* status);
+// The spectrum of a chirp of nc samples at block length n, in the block kernel's order, into d_h (room for n + nc).
+int rc_block_spectrum(asarf_ctx* ctx, const float* chirp_iq, int nc, int n, float2* d_h);
+// True when the padded chirp has no sample past its first nc (its correlation then needs no more than them).
+bool chirp_tail_zero(const float* chirp_iq, int nc, int n);
 int get_col_split(asarf_ctx* ctx, int n, ColSplit* out, int n2_max = 0);
 // Column-transform launch arguments: element m of group g is read from row g*in_g + m*in_m, element k written
 // to row g*out_g + k*out_m; twf (nullptr = none) is the inter-pass twiddle table.

@@ -868,6 +868,11 @@ __global__ __launch_bounds__(64) void k_finalize(FinalizeArgs f) {
         c.sin_corr = (float)delta;
         c.inv_cos = (float)(1.0 / cosc);
         c.identity = 0;
+        c.ii = (float)ca;
+        c.i0 = (float)cb;
+        c.qi = (float)cc;
+        c.qq = (float)cd;
+        c.q0 = (float)ce;
         r->coef = c;
         r->nblocks = f.nblocks;
         r->dc_poly[0] = poly[0];

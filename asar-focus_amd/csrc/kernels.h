@@ -93,10 +93,12 @@ __device__ __forceinline__ void fbaq4_row_decode(const unsigned char* rec, long 
     }
 }
 
-// Affine I/Q correction: I' = (I - dc_i) * inv_gain, Q' = (Q - dc_q - I' * sin_corr) * inv_cos.
+// Affine I/Q correction: I' = (I - dc_i) * inv_gain, Q' = (Q - dc_q - I' * sin_corr) * inv_cos, and the same as one
+// affine map, I' = ii I + i0, Q' = qi I + qq Q + q0 (set by k_finalize in FP64; the block range compression uses it).
 struct IqCoef {
     float dc_i, dc_q, inv_gain, sin_corr, inv_cos;
     int identity;
+    float ii, i0, qi, qq, q0;
 };
 
 // Device-resident results of the fused statistics/Doppler stage.
@@ -148,6 +150,15 @@ struct RcArgs {
     int no_static;      // use the runtime-radix kernel even where a compile-time kernel exists (autotuner)
     int static_variant; // which compile-time variant of the length (autotuner; 0 = default)
     LinesDesc lines;    // RAW_ERS_LINES, RAW_ASAR_FBAQ4
+    // block kernels (rc_block.h): hconj holds the block length's spectrum in pairs (launch_rc_block_spectrum)
+    const float4* rc_tw; // twiddles of every pass, in pairs
+    int blocks;          // blocks per line
+    int block_step;      // output samples per block
+};
+
+// Range compression in blocks of a line: transform length, blocks per line, kept samples per block.
+struct RcBlock {
+    int n, blocks, step;
 };
 
 struct ColFftArgs {
@@ -343,6 +354,15 @@ int range_compress_static_variants(int n);
 // Padded-layout range compression (k_rc_pad.hip): variants per length and their launcher.
 int range_compress_pad_variants(int n);
 bool launch_range_compress_pad(const RcArgs& a, int fmt, int variant, hipStream_t s, hipError_t* err);
+// Range compression in blocks (k_rc_block.hip): the block length for lines of nr samples and a chirp of nc (single:
+// one block per line, for in-place lines; only > 0: that length; false when no compiled length suits), its radices,
+// the launch.
+bool rc_block_choose(int nr, int nc, bool single, RcBlock* out, int only = 0);
+int rc_block_radices(int n, int* radices);
+hipError_t launch_rc_block(const RcArgs& a, int fmt, int n, hipStream_t s);
+// The spectrum conj(FFT_n(chirp)) / n of a chirp of nc samples (device) in the order the kernel's lanes read it: bin
+// j + (2 s + e) m at out[2 (s m + j) + e], m = n / (last radix).
+hipError_t launch_rc_block_spectrum(const float2* chirp, int nc, int n, float2* out, hipStream_t s);
 hipError_t launch_col_fft(const ColFftArgs& a, bool inverse, hipStream_t s);
 hipError_t launch_rc_mfma(const RcArgs& a, int raw_format, hipStream_t s);
 hipError_t launch_row_mfma(const RowFftArgs& a, bool inverse, hipStream_t s);

@@ -53,6 +53,10 @@ struct asarf_plan {
     hipEvent_t ev_fork = nullptr, ev_join = nullptr;
     std::vector<hipEvent_t> ev_core;
     float2* hconj = nullptr;
+    // range compression in blocks of a line (rc_block.h; n = 0: by transforms of the padded line)
+    RcBlock rcb{};
+    float2* hblk = nullptr;
+    const float4* rc_tw = nullptr;
     ColConst* col = nullptr;
     long long* partials = nullptr;
     long long* totals = nullptr;
@@ -100,7 +104,7 @@ static int plan_alloc(asarf_plan* pl, void** p, size_t bytes) {
 }
 
 static void plan_free(asarf_plan* pl) {
-    void* bufs[] = {pl->img,    pl->img2, pl->hconj, pl->col, pl->partials, pl->totals,
+    void* bufs[] = {pl->img,    pl->img2, pl->hconj, pl->hblk, pl->col, pl->partials, pl->totals,
                     pl->corr,   pl->res,  pl->ml,    pl->rsl, pl->fbaq_lut, pl->gr_r0, pl->gr_fx, pl->gr_start};
     for (void* b : bufs)
         if (b) (void)hipFree(b);
@@ -265,6 +269,19 @@ extern "C" int asarf_plan_create(asarf_ctx* c, const asarf_focus_params* p, cons
         a.plan = pl->rplan->dev();
         if (launch_row_fft(a, true, c->stream) != hipSuccess)
             return fail(set_error(ASARF_EHIP, "asarf_plan_create: chirp transform"));
+    }
+    // Lines are compressed in blocks when the chirp ends within its nc samples and a compiled block length suits
+    // (any line length does; see k_rc_block.hip). ASARF_RC_BLOCK=0 keeps the transforms of the padded line,
+    // ASARF_RC_BLOCK=<n> takes block length n (comparison runs and tests).
+    const char* rb_env = std::getenv("ASARF_RC_BLOCK");
+    if (!(rb_env && rb_env[0] == '0') && chirp_tail_zero(chirp_iq, p->nc, nrp) &&
+        rc_block_choose(p->nr, p->nc, false, &pl->rcb, rb_env ? std::atoi(rb_env) : 0)) {
+        pl->rc_tw = get_rc_twiddles(c, pl->rcb.n, &st);
+        if (!pl->rc_tw) return fail(st);
+        if ((st = plan_alloc(pl, (void**)&pl->hblk, sizeof(float2) * (size_t)(pl->rcb.n + p->nc)))) return fail(st);
+        if ((st = rc_block_spectrum(c, chirp_iq, p->nc, pl->rcb.n, pl->hblk)) != ASARF_OK) return fail(st);
+    } else {
+        pl->rcb = RcBlock{};
     }
     // results window (main_flow.cc:155-201) for both signs of the Doppler constant term
     const int max_ap = aperture_pixels_max(p->wavelength, p->prf, p->az_bandwidth_fraction, p->vr_poly,
@@ -472,22 +489,32 @@ static int enqueue_to_spectrum(asarf_plan* pl, const void* raw, bool core_path) 
     ra.nrv = pl->nrv;
     ra.zero_to = pl->nrv;
     ra.coef = &pl->res->coef;
-    ra.hconj = pl->hconj;
-    ra.plan = pl->rplan->dev();
-    ra.mfma = pl->fft_mfma;
     ra.lines = pl->lines;
-    {
-        const auto t = c->tuned_rows.find(pl->nrp);
-        ra.no_static = (t != c->tuned_rows.end() && !t->second.use_static) ? 1 : 0;
-        ra.static_variant = (t != c->tuned_rows.end()) ? t->second.static_variant : 0;
-        // ASARF_RC_VARIANT=<v> forces compile-time variant v (comparison runs and tests)
-        const char* v_env = std::getenv("ASARF_RC_VARIANT");
-        if (v_env && range_compress_static_variants(pl->nrp) > 0) {
+    // A saved or measured choice of the autotuner other than the default, or ASARF_RC_VARIANT=<v> (comparison runs
+    // and tests), runs the transforms of the padded line.
+    const auto t = c->tuned_rows.find(pl->nrp);
+    const bool tuned_static = t == c->tuned_rows.end() || t->second.use_static;
+    const int tuned_variant = t == c->tuned_rows.end() ? 0 : t->second.static_variant;
+    const char* v_env = std::getenv("ASARF_RC_VARIANT");
+    const bool forced = v_env && range_compress_static_variants(pl->nrp) > 0;
+    if (pl->rcb.n > 0 && !pl->fft_mfma && !forced && tuned_static && tuned_variant == 0) {
+        ra.hconj = pl->hblk;
+        ra.rc_tw = pl->rc_tw;
+        ra.blocks = pl->rcb.blocks;
+        ra.block_step = pl->rcb.step;
+        HIP_CHECK(launch_rc_block(ra, p.raw_format, pl->rcb.n, s));
+    } else {
+        ra.hconj = pl->hconj;
+        ra.plan = pl->rplan->dev();
+        ra.mfma = pl->fft_mfma;
+        ra.no_static = tuned_static ? 0 : 1;
+        ra.static_variant = tuned_variant;
+        if (forced) {
             ra.no_static = 0;
             ra.static_variant = std::atoi(v_env) % range_compress_static_variants(pl->nrp);
         }
+        HIP_CHECK(launch_range_compress(ra, p.raw_format, s));
     }
-    HIP_CHECK(launch_range_compress(ra, p.raw_format, s));
     ST_CHECK(mark(pl, "range_compression"));
     // 3. azimuth FFT (permuted bins), rows >= Na read as zero; with two passes, A img -> img2 and B img2 -> img
     // (out of place streams faster than in place)

@@ -1,7 +1,8 @@
 // Autotuner: measures candidate transform schedules on the device and records the fastest per length in the
 // context, where the planner (get_plan, get_col_split) and the plans created afterwards pick them up.
-//   rows (range compression): the compile-time variants where the length has them (radix sequences and lanes
-//     per line), and runtime-radix plans with the factors of the length in different orders and groupings;
+//   rows (range compression): the block kernels (the default of every length, recorded as variant 0), the
+//     compile-time variants where the length has them (radix sequences and lanes per line), and runtime-radix plans
+//     with the factors of the length in different orders and groupings;
 //   columns (azimuth): every two-pass split n1 x n2 (and the single pass where it fits LDS).
 // Timing: one warm-up launch, then the minimum of `reps` launches bracketed by HIP events.
 #include <algorithm>
@@ -101,21 +102,26 @@ extern "C" int asarf_autotune_fft(asarf_ctx* c, int n, int layout, int batch, in
     if (layout == ASARF_FFT_ROWS) {
         // range compression of `batch` lines of zero-valued raw bytes into an n-wide image
         const int nr_in = n / 2;
+        // the block kernels compress the lines this transform length pads: 11/12 samples, 1/12 chirp
+        RcBlock rb{};
+        const int blk_nc = std::max(1, n / 12), blk_nr = n - blk_nc;
+        const bool block = blk_nr > blk_nc && rc_block_choose(blk_nr, blk_nc, false, &rb);
         void* raw = nullptr;
         float2 *img = nullptr, *h = nullptr;
-        HIP_CHECK(hipMalloc(&raw, (size_t)batch * nr_in * 2));
+        const size_t raw_bytes = (size_t)batch * (block ? blk_nr : nr_in) * 2;
+        HIP_CHECK(hipMalloc(&raw, raw_bytes));
         auto cleanup = [&]() {
             (void)hipFree(raw);
             if (img) (void)hipFree(img);
             if (h) (void)hipFree(h);
         };
         if (hipMalloc(&img, sizeof(float2) * (size_t)batch * n) != hipSuccess ||
-            hipMalloc(&h, sizeof(float2) * (size_t)n) != hipSuccess) {
+            hipMalloc(&h, sizeof(float2) * (size_t)std::max(n, rb.n)) != hipSuccess) {
             cleanup();
             return set_error(ASARF_ENOMEM, "asarf_autotune_fft: buffers");
         }
-        (void)hipMemsetAsync(raw, 0, (size_t)batch * nr_in * 2, s);
-        (void)hipMemsetAsync(h, 0, sizeof(float2) * (size_t)n, s);
+        (void)hipMemsetAsync(raw, 0, raw_bytes, s);
+        (void)hipMemsetAsync(h, 0, sizeof(float2) * (size_t)std::max(n, rb.n), s);
         std::vector<std::vector<int>> cands = row_candidates(n, kRowThreads);
         std::vector<const FftPlanHost*> plans;
         float2* tw = get_twiddles(c, n, &st);
@@ -131,8 +137,9 @@ extern "C" int asarf_autotune_fft(asarf_ctx* c, int n, int layout, int batch, in
             plans.push_back(p.get());
             c->plans[std::make_pair(n, -1000 - c->tune_key++)] = std::move(p);
         }
-        // candidates -1 .. -nv: the compile-time variants of the length (if any)
-        const int nv = range_compress_static_variants(n);
+        // candidate -1: the block kernels; -1 (without them) or -2 .. -nv: the compile-time variants of the length
+        const float4* rc_tw = block ? get_rc_twiddles(c, rb.n, &st) : nullptr;
+        const int nv = std::max(range_compress_static_variants(n), rc_tw ? 1 : 0);
         for (int ci = -nv; ci < (int)plans.size(); ++ci) {
             RcArgs a{};
             a.in = raw;
@@ -157,12 +164,22 @@ extern "C" int asarf_autotune_fft(asarf_ctx* c, int n, int layout, int batch, in
             a.plan = pd;
             a.no_static = ci >= 0;
             a.static_variant = ci < 0 ? -1 - ci : 0;
-            hipError_t e = launch_range_compress(a, RAW_U8, s);
+            if (ci == -1 && rc_tw) {
+                a.in_stride = a.nr_in = blk_nr;
+                a.nrv = a.zero_to = blk_nr - blk_nc;
+                a.rc_tw = rc_tw;
+                a.blocks = rb.blocks;
+                a.block_step = rb.step;
+            }
+            auto launch = [&]() {
+                return a.rc_tw ? launch_rc_block(a, RAW_U8, rb.n, s) : launch_range_compress(a, RAW_U8, s);
+            };
+            hipError_t e = launch();
             if (e != hipSuccess) continue;  // candidate not launchable (e.g. LDS): skip
             float ms_min = INFINITY;
             for (int k = 0; k < reps; ++k) {
                 (void)hipEventRecord(t.a, s);
-                (void)launch_range_compress(a, RAW_U8, s);
+                (void)launch();
                 (void)hipEventRecord(t.b, s);
                 (void)hipEventSynchronize(t.b);
                 float ms = 0.f;
