@@ -827,7 +827,6 @@ extern "C" int asarf_range_doppler(asarf_ctx* c, const asarf_rda_params* p, asar
     ColConstArgs ca{};
     ca.col = col;
     ca.nrv = nrv;
-    ca.dc_poly = nullptr;  // by value
     for (int i = 0; i < 3; ++i) ca.dc_val[i] = p->dc_poly[i];
     ca.clear_reach = 1;
     for (int i = 0; i < 3; ++i) ca.vr_poly[i] = p->vr_poly[i];

@@ -6,6 +6,7 @@
 // sin(pi d)/pi cancels in the normalisation, so no transcendental is evaluated per tap (sinc16_interp).
 // The matched filter follows range_doppler_algorithm.cu:197-309 with FP64 geometry and phase (reduced to turns
 // before the hardware sine/cosine, whose argument is in turns).
+#include "col_const.h"
 #include "interp.h"
 #include "kernels.h"
 #include "poly.h"
@@ -30,30 +31,7 @@ static RcmcArgs with_window(const RcmcArgs& in) {
 
 __global__ void k_col_const(ColConstArgs a) {
     const int x = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool valid = x < a.nrv;
-    int r = 0;
-    if (valid) {
-        const double step = a.prf / (double)a.nbins;
-        const double dc = polyval(a.dc_poly ? a.dc_poly : a.dc_val, 3, (double)x);
-        const double r0 = a.r_first + (double)x * a.range_spacing;
-        const double vr = polyval(a.vr_poly, 3, (double)x);
-        ColConst c;
-        c.dc = dc;
-        c.dc_off = round(dc / step) * step;
-        c.shift_k = a.wavelength * a.wavelength * r0 / (8.0 * vr * vr * a.range_spacing);
-        c.inv_ka = a.wavelength * r0 / (2.0 * vr * vr);
-        a.col[x] = c;
-        // The aliased bin frequency stays within prf/2 of the centroid, so |f| <= prf/2 + |dc| bounds the
-        // shift of every bin (plus one pixel against rounding).
-        const double fmax = (0.5 * a.prf + fabs(dc)) * (1.0 + 1e-12);
-        const double smax = c.shift_k * fmax * fmax;
-        r = (smax >= 0.0 && smax < 1e6) ? (int)floor(smax + 0.5) + 1 : 1000000;
-    }
-    if (a.reach) {
-        // one atomic per wave; every lane of the wave takes part in the reduction
-        for (int o = 32; o > 0; o >>= 1) r = max(r, __shfl_xor(r, o));
-        if ((threadIdx.x & 63) == 0 && r > 0) atomicMax(a.reach, r);
-    }
+    col_const_store(a, x, a.dc_val);
 }
 
 // Clears the RCMC shift bound before k_col_const takes its maximum (a one-lane vector store; no memset, so the

@@ -10,6 +10,7 @@
 //    correction is affine, so the corrected lag-1 sum of every block is a bilinear form in these sums; one FP64
 //    finalisation wave turns them into the DC bias, gain, phase correction, block Doppler estimates and the
 //    degree-2 Doppler polynomial without a second read of the raw data.
+#include "col_const.h"
 #include "kernels.h"
 #include "poly.h"
 
@@ -185,11 +186,11 @@ __device__ __forceinline__ T wave_sum(T v) {
     return v;
 }
 
-// Workgroup (tile, strip): lane t owns columns [V*(256*tile + t), +V) over rows [128*strip, +128) and
+// Workgroup (tile, strip): lane t owns columns [V*(256*tile + t), +V) over the strip's rows (at most 128) and
 // accumulates exact integer sums; lag-1 products pair each row with the one above (the strip re-reads its
 // preceding row). With V = 4 a row of a lane is one 8-byte load (4 I/Q byte pairs). Statistics are reduced over
 // the workgroup; lag sums per Doppler block (slot = block - first block of the tile) through per-column LDS rows.
-// Integer ranges: a column's sums over 128 rows stay below 128 * 255^2 < 2^31.
+// Integer ranges: a column's sums over at most 128 rows stay below 128 * 255^2 < 2^31.
 // LINES: the rows are ERS level-0 lines (RawMomentsArgs::lines): row y of range column x holds line sample
 // x - shift(y) when that is one of the line's samples, else NaN, which the statistics skip and the lag-1 sums treat
 // as the zero ZeroNaNs makes it (a pair counts only when both of its samples are valid). V = 4 needs the shifts
@@ -201,8 +202,8 @@ __global__ __launch_bounds__(kThreads) void k_raw_moments(RawMomentsArgs a) {
     const int tile = blockIdx.x;
     const int strip = blockIdx.y;
     const int x0 = (tile * kThreads + threadIdx.x) * V;
-    const int y0 = strip * kStripRows;
-    const int y1 = min(y0 + kStripRows, a.na);
+    const int y0 = strip * a.strip_rows;
+    const int y1 = min(y0 + a.strip_rows, a.na);
     const unsigned char* raw = static_cast<const unsigned char*>(a.raw);
     const int nv = min(V, max(0, a.nr - x0));  // valid columns of this lane: V or 0 (nr % V == 0)
     int st[5] = {0, 0, 0, 0, 0};
@@ -356,8 +357,8 @@ __global__ __launch_bounds__(kThreads) void k_raw_moments8(RawMomentsArgs a) {
     const int tile = blockIdx.x;
     const int strip = blockIdx.y;
     const int x0 = (tile * kThreads + threadIdx.x) * V;
-    const int y0 = strip * kStripRows;
-    const int y1 = min(y0 + kStripRows, a.na);
+    const int y0 = strip * a.strip_rows;
+    const int y1 = min(y0 + a.strip_rows, a.na);
     const bool valid = x0 < a.nr;  // nr % 8 == 0: all eight columns of the lane, or none
     const unsigned char* raw = static_cast<const unsigned char*>(a.raw);
     auto load_row = [&](int y) -> uint4 { return *reinterpret_cast<const uint4*>(raw + ((long)y * a.nr + x0) * 2); };
@@ -524,8 +525,8 @@ __global__ __launch_bounds__(kThreads) void k_raw_moments_fbaq(RawMomentsArgs a)
     const int tile = blockIdx.x;
     const int strip = blockIdx.y;
     const int x = tile * kThreads + threadIdx.x;
-    const int y0 = strip * kStripRows;
-    const int y1 = min(y0 + kStripRows, a.na);
+    const int y0 = strip * a.strip_rows;
+    const int y1 = min(y0 + a.strip_rows, a.na);
     const bool col_ok = x < a.nr;
     const unsigned char* base = static_cast<const unsigned char*>(a.raw);
     const LinesDesc L = a.lines;
@@ -701,6 +702,7 @@ __global__ __launch_bounds__(kThreads) void k_reduce_raw(RawReduceArgs a) {
             return bits;
     };
     const int v = blockIdx.x;
+    if (v == 0 && threadIdx.x == 0 && a.clear) *a.clear = 0;  // the RCMC shift bound, before k_finalize raises it
     const int nval = kRawStats + a.nslots * kRawLag;
     T acc = 0;
     if (v < kRawStats) {
@@ -753,55 +755,21 @@ hipError_t launch_reduce_raw(const RawReduceArgs& a, hipStream_t s) {
     return hipGetLastError();
 }
 
-// Degree-M-1 least squares on one wave (lane i owns point i, n <= 64): Householder QR with wave reductions,
-// the same steps as polyfit_qr (util/src/math_utils.cc:23-44), result highest power first.
-template <int M>
-__device__ bool polyfit_wave(double x, double y, int n, double* out) {
+// Degree-2 least squares of n equispaced samples on one wave: lane b holds y at x = b * step + x0. On the centred index
+// u = b - (n - 1) / 2 the polynomials 1, u, u^2 - (n^2 - 1) / 12 are orthogonal, so the fit is three independent sums
+// (the reference solves the same problem by QR, util/src/math_utils.cc:23-44, whose steps depend on each other: 12
+// reductions in a row). Result highest power of x first.
+__device__ __forceinline__ void polyfit2_equispaced(double y, int n, double x0, double step, double* out) {
     const int lane = threadIdx.x & 63;
-    const bool in = lane < n;
-    double a[M];
-    double v = 1.0;
-#pragma unroll
-    for (int c = 0; c < M; ++c) {
-        a[c] = in ? v : 0.0;
-        v *= x;
-    }
-    double b = in ? y : 0.0;
-    double rdiag[M], rrow[M][M];
-#pragma unroll
-    for (int k = 0; k < M; ++k) {
-        const double ak = lane >= k ? a[k] : 0.0;
-        const double nrm = sqrt(wave_sum(ak * ak));
-        if (nrm == 0.0) return false;
-        const double akk = __shfl(a[k], k, 64);
-        const double alpha = akk > 0.0 ? -nrm : nrm;
-        const double hv = (lane == k) ? ak - alpha : ak;  // Householder vector (zero above row k)
-        const double vv = wave_sum(hv * hv);
-#pragma unroll
-        for (int c = k + 1; c < M; ++c) {
-            const double d = wave_sum(hv * a[c]);
-            a[c] -= 2.0 * d / vv * hv;
-        }
-        const double d = wave_sum(hv * b);
-        b -= 2.0 * d / vv * hv;
-        rdiag[k] = alpha;
-#pragma unroll
-        for (int c = k + 1; c < M; ++c) rrow[k][c] = __shfl(a[c], k, 64);
-    }
-    double qb[M];
-#pragma unroll
-    for (int k = 0; k < M; ++k) qb[k] = __shfl(b, k, 64);
-    double coef[M];
-#pragma unroll
-    for (int k = M - 1; k >= 0; --k) {
-        double t = qb[k];
-#pragma unroll
-        for (int c = k + 1; c < M; ++c) t -= rrow[k][c] * coef[c];
-        coef[k] = t / rdiag[k];
-    }
-#pragma unroll
-    for (int k = 0; k < M; ++k) out[k] = coef[M - 1 - k];
-    return true;
+    const double nn = (double)n, mid = 0.5 * (nn - 1.0), m2 = (nn * nn - 1.0) / 12.0;
+    const double u = (double)lane - mid, q = u * u - m2, v = lane < n ? y : 0.0;
+    const double s0 = wave_sum(v), s1 = wave_sum(u * v), s2 = wave_sum(q * v);
+    const double c0 = s0 / nn, c1 = s1 / (nn * m2), c2 = s2 * 15.0 / (nn * m2 * (nn * nn - 4.0));
+    // u = (x - xm) / step with xm = x0 + mid * step
+    const double xm = x0 + mid * step;
+    out[0] = c2 / (step * step);
+    out[1] = c1 / step - 2.0 * xm * out[0];
+    out[2] = c0 - c2 * m2 - xm * (c1 / step - xm * out[0]);
 }
 
 // One-wave FP64 finalisation of the fused statistics. With the corrected sample u = a I + b, v = c I + d Q + e,
@@ -809,8 +777,9 @@ __device__ bool polyfit_wave(double x, double y, int n, double* out) {
 //   sum conj(s_prev) s_cur = sum(u1 u2 + v1 v2) + i sum(u1 v2 - v1 u2),
 // each term expanded over the raw lag moments. Padding columns of the last block (Q4) hold the corrected image
 // of raw 0 when the correction runs over the padded width (Q1), i.e. the constant (b, e). Lane b handles block b.
-__global__ __launch_bounds__(64) void k_finalize(FinalizeArgs f) {
-    const int lane = threadIdx.x;
+__device__ __forceinline__ void finalize_wave(const FinalizeArgs& f, double* dc3) {
+    const int lane = threadIdx.x & 63;
+    const bool store = blockIdx.x == 0;
     const long long* T = f.totals;
     // exact integer sums, or (FBAQ-4 records) FP64 sums stored as bit patterns
     auto tot = [&](int i) -> double { return f.f64 ? __longlong_as_double(T[i]) : (double)T[i]; };
@@ -849,12 +818,15 @@ __global__ __launch_bounds__(64) void k_finalize(FinalizeArgs f) {
         if (q1 && pad1 > pad0 && f.na > 1) re += (double)(f.na - 1) * (double)(pad1 - pad0) * (cb * cb + ce * ce);
         bx = (double)((xb + xe) / 2);
         by = f.prf * atan2(im, re) / (2.0 * kPi);
-        r->block_freq[lane] = by;
-        r->block_x[lane] = bx;
+        if (store) {
+            r->block_freq[lane] = by;
+            r->block_x[lane] = bx;
+        }
     }
     double poly[3];
-    if (!polyfit_wave<3>(bx, by, f.nblocks, poly)) poly[0] = poly[1] = poly[2] = 0.0;
-    if (lane == 0) {
+    polyfit2_equispaced(by, f.nblocks, (double)(f.step / 2), (double)f.step, poly);
+    if (lane < 3) dc3[lane] = poly[lane];
+    if (lane == 0 && store) {
         r->dc_i = dci;
         r->dc_q = dcq;
         r->stddev_i = sqrt((SII - 2.0 * dci * SI + nvalid * dci * dci) / ntot);
@@ -884,12 +856,21 @@ __global__ __launch_bounds__(64) void k_finalize(FinalizeArgs f) {
         const int in_rows = pos ? f.imp_in_rows_pos : f.imp_in_rows_neg;
         r->imp_rows = (f.ml_ratio > 0.f) ? (int)roundf((float)in_rows / f.ml_ratio) : 0;
         r->pad = in_rows;
-        r->rcmc_reach = 0;
     }
 }
 
-hipError_t launch_finalize(const FinalizeArgs& a, hipStream_t s) {
-    hipLaunchKernelGGL(k_finalize, dim3(1), dim3(64), 0, s, a);
+// Every workgroup's first wave finalises (the sums are a few KB in L2; the chain is latency, not work), then its lanes
+// compute the range-Doppler constants of its columns from the polynomial (col_const.h): one launch for both, without a
+// hand-over between workgroups. Workgroup 0 stores the results.
+__global__ __launch_bounds__(kThreads) void k_finalize(FinalizeArgs f, ColConstArgs ca) {
+    __shared__ double dc3[3];
+    if (threadIdx.x < 64) finalize_wave(f, dc3);
+    __syncthreads();
+    col_const_store(ca, blockIdx.x * kThreads + threadIdx.x, dc3);
+}
+
+hipError_t launch_finalize(const FinalizeArgs& a, const ColConstArgs& ca, hipStream_t s) {
+    hipLaunchKernelGGL(k_finalize, dim3((ca.nrv + kThreads - 1) / kThreads), dim3(kThreads), 0, s, a, ca);
     return hipGetLastError();
 }
 

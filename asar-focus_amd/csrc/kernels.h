@@ -14,7 +14,7 @@ constexpr int kThreads = 256;      // generic kernels and column transforms
 constexpr int kRowThreads = 512;   // row transforms: one row per workgroup
 constexpr int kColTile = 16;   // columns per workgroup in column transforms (16 x 8 B = one 128 B line)
 constexpr int kMaxE = 16;      // complex elements per lane in a Stockham pass
-constexpr int kStripRows = 128; // rows per workgroup in the raw statistics pass
+constexpr int kStripRows = 128; // most rows per workgroup in the raw statistics pass
 constexpr int kRawStats = 6;    // SI, SQ, SII, SQQ, SIQ, N
 constexpr int kRawLag = 9;      // LII, LQQ, LIQ, LQI, LI1, LQ1, LI2, LQ2, M per Doppler block
 constexpr int kMaxDcBlocks = 64;
@@ -234,6 +234,7 @@ struct RawMomentsArgs {
     int ntiles;       // tiles of 256*vec columns
     int nslots;       // Doppler blocks a tile can touch: (256*vec - 1)/step + 2
     int nstrips;
+    int strip_rows;   // rows per strip (<= kStripRows)
     long long* partials; // [strip][tile][kRawStats + nslots*kRawLag]
     long long* corr;     // vec 8: [nstrips][nblocks][kRawLag] lag sums of the odd block-start columns (written for
                          // odd starts only)
@@ -247,6 +248,7 @@ struct RawReduceArgs {
     const long long* corr;  // vec 8: straddle-column lag sums ([nstrips][nblocks][kRawLag]) to move between
                             // neighbouring blocks (else null)
     long long* totals;  // [kRawStats + nblocks*kRawLag]
+    int* clear;         // set to 0 (the RCMC shift bound that k_finalize maximises), or null
     int f64;            // partials and totals hold FP64 sums (bit patterns in the int64 slots): RAW_ASAR_FBAQ4
 };
 
@@ -267,8 +269,7 @@ struct FinalizeArgs {
 struct ColConstArgs {
     ColConst* col;
     int nrv;
-    const double* dc_poly;  // device; nullptr: dc_val
-    double dc_val[3];       // the Doppler polynomial by value (host callers)
+    double dc_val[3];       // the Doppler polynomial (k_col_const; k_finalize takes the one it fitted)
     double vr_poly[3];
     double wavelength, range_spacing, r_first, prf;
     int nbins;
@@ -390,7 +391,8 @@ hipError_t launch_dc_cf32(const float2* img, long stride, int ys, int x_begin0, 
 hipError_t launch_reduce_f64(const double* partials, int nparts, int nvals, double* totals, hipStream_t s);
 hipError_t launch_raw_moments(const RawMomentsArgs& a, int raw_format, hipStream_t s);
 hipError_t launch_reduce_raw(const RawReduceArgs& a, hipStream_t s);
-hipError_t launch_finalize(const FinalizeArgs& a, hipStream_t s);
+// FP64 finalisation of the statistics and the column constants (from the polynomial it fits; ca.dc_val unused).
+hipError_t launch_finalize(const FinalizeArgs& a, const ColConstArgs& ca, hipStream_t s);
 hipError_t launch_multilook(const MultilookArgs& a, hipStream_t s);
 hipError_t launch_rsl(float* img, int nr, int rows, const float* tab, hipStream_t s);
 hipError_t launch_srgr(const SrgrArgs& a, hipStream_t s);

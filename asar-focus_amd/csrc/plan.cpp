@@ -38,12 +38,15 @@ struct asarf_plan {
     asarf_focus_params p{};
     int nrp = 0, nap = 0, nrv = 0;
     long stride = 0;
-    int nblocks = 0, step = 0, nstrips = 0, raw_vec = 1;  // raw_vec: widest column count per lane the rows allow
-    const FftPlanHost* rplan = nullptr;
+    int nblocks = 0, step = 0, nstrips = 0, strip_rows = 0;
+    int raw_vec = 1;  // widest column count per lane the rows allow
+    const FftPlanHost* rplan = nullptr;  // with hconj: the transform of the padded line (padded_spectrum)
+    std::vector<float> chirp;            // kept until hconj exists
     ColSplit cs;
     // device buffers
     float2* img = nullptr;
     float2* img2 = nullptr;  // second image: out-of-place target of the column passes and of the RCMC stage
+    bool core_certain = false;  // no Doppler estimate of this radar exceeds the core's halo (doppler_reach_bound)
     bool core = false;       // fused azimuth core: pass B + RCMC + matched filter + pass B' in one kernel
     // Column chunks of the azimuth tail (core, then in-place pass A', per chunk) alternating between the context's
     // stream and a second stream, each chunk's core after the previous chunk's: one chunk's pass A' (HBM-bound)
@@ -97,6 +100,47 @@ static void raw_tiles(const asarf_plan* pl, int vec, int* ntiles, int* nslots) {
     *nslots = (tw - 1) / pl->step + 2;
 }
 
+// Bound on the RCMC shift (DevResults::rcmc_reach) over every Doppler polynomial the statistics can yield. The block
+// estimates lie within +-prf/2 (an arctangent), so the fitted polynomial at column x lies within prf/2 times the sum of
+// |w_b(x)| over the fit's weights on the blocks (2.2 at the ends, 1.3 in the middle). Evaluated at the ends of 64
+// intervals of columns and bounded inside them: a sum of absolute quadratics exceeds its chord's larger end by at most
+// K h^2 / 8 with K the sum of their |second derivatives|, and Vr, one quadratic, falls below its smaller end by at most
+// |a| h^2 / 4.
+static int doppler_reach_bound(const asarf_focus_params& p, int nblocks, int step, int nrv) {
+    const int n = nblocks;
+    if (n < 3) return 1000000;
+    const double nn = n, mid = 0.5 * (nn - 1.0), m2 = (nn * nn - 1.0) / 12.0;
+    const double s2 = nn * m2, s4 = nn * m2 * (nn * nn - 4.0) / 15.0;
+    double curv = 0.0;
+    for (int b = 0; b < n; ++b) curv += std::fabs(2.0 * ((b - mid) * (b - mid) - m2) / s4);
+    auto lambda = [&](double x) {
+        const double u = (x - step / 2) / step - mid, q = u * u - m2;
+        double sum = 0.0;
+        for (int b = 0; b < n; ++b) {
+            const double ub = b - mid;
+            sum += std::fabs(1.0 / nn + u * ub / s2 + q * (ub * ub - m2) / s4);
+        }
+        return sum;
+    };
+    const int parts = 64;
+    const double h = (double)nrv / parts, hu = h / step;
+    double worst = 0.0;
+    double l0 = lambda(0.0), v0 = polyval(p.vr_poly, 3, 0.0);
+    for (int i = 1; i <= parts; ++i) {
+        const double x1 = i * h, l1 = lambda(x1), v1 = polyval(p.vr_poly, 3, x1);
+        const double lam = std::max(l0, l1) + curv * hu * hu / 8.0;
+        const double vr = std::min(v0, v1) - std::fabs(p.vr_poly[0]) * h * h / 4.0;
+        if (!(vr > 0.0)) return 1000000;
+        const double r0 = p.slant_range_first + x1 * p.range_spacing;
+        const double f = 0.5 * p.prf * (1.0 + lam);
+        const double s = p.wavelength * p.wavelength * r0 / (8.0 * vr * vr * p.range_spacing) * f * f;
+        worst = std::max(worst, s * (1.0 + 1e-9));
+        l0 = l1;
+        v0 = v1;
+    }
+    return worst < 1e6 ? (int)std::floor(worst + 0.5) + 1 : 1000000;
+}
+
 static int plan_alloc(asarf_plan* pl, void** p, size_t bytes) {
     HIP_CHECK(hipMalloc(p, bytes));
     pl->bytes += bytes;
@@ -113,6 +157,46 @@ static void plan_free(asarf_plan* pl) {
     if (pl->ev_fork) (void)hipEventDestroy(pl->ev_fork);
     if (pl->ev_join) (void)hipEventDestroy(pl->ev_join);
     if (pl->s1) (void)hipStreamDestroy(pl->s1);
+}
+
+// Whether an execution transforms padded lines: without a block length, for split-bfloat16 transforms, for a saved or
+// measured choice of the autotuner other than the default, or with ASARF_RC_VARIANT=<v> (comparison runs and tests).
+static bool padded_lines(const asarf_plan* pl) {
+    const auto t = pl->ctx->tuned_rows.find(pl->nrp);
+    const bool tuned = t != pl->ctx->tuned_rows.end() && (!t->second.use_static || t->second.static_variant != 0);
+    const bool forced = std::getenv("ASARF_RC_VARIANT") && range_compress_static_variants(pl->nrp) > 0;
+    return pl->rcb.n == 0 || pl->fft_mfma || tuned || forced;
+}
+
+// The padded line's transform and the chirp spectrum conj(FFT(chirp))/nrp (inverse-direction transform of the
+// conjugated chirp), built when first needed.
+static int padded_spectrum(asarf_plan* pl) {
+    if (pl->hconj) return ASARF_OK;
+    const int nrp = pl->nrp;
+    int st = ASARF_OK;
+    pl->rplan = get_plan(pl->ctx, nrp, kRowThreads, &st);
+    if (!pl->rplan) return st;
+    std::vector<float2> h(nrp);
+    for (int i = 0; i < nrp; ++i) h[i] = make_float2(pl->chirp[2 * i], -pl->chirp[2 * i + 1]);
+    float2* d = nullptr;
+    ST_CHECK(plan_alloc(pl, (void**)&d, sizeof(float2) * (size_t)nrp));
+    RowFftArgs a{};
+    a.in = d;
+    a.in_stride = nrp;
+    a.out = d;
+    a.out_stride = nrp;
+    a.rows = 1;
+    a.scale = 1.0f / (float)nrp;
+    a.plan = pl->rplan->dev();
+    if (hipMemcpy(d, h.data(), sizeof(float2) * (size_t)nrp, hipMemcpyHostToDevice) != hipSuccess ||
+        launch_row_fft(a, true, pl->ctx->stream) != hipSuccess) {
+        (void)hipFree(d);
+        pl->bytes -= sizeof(float2) * (size_t)nrp;
+        return set_error(ASARF_EHIP, "asarf_plan: chirp spectrum of %d samples", nrp);
+    }
+    pl->hconj = d;
+    std::vector<float>().swap(pl->chirp);
+    return ASARF_OK;
 }
 
 extern "C" int asarf_plan_create(asarf_ctx* c, const asarf_focus_params* p, const float* chirp_iq, asarf_plan** out) {
@@ -179,15 +263,31 @@ extern "C" int asarf_plan_create(asarf_ctx* c, const asarf_focus_params* p, cons
                           ? 4
                           : 1;
     if (p->raw_format == ASARF_RAW_ASAR_FBAQ4) pl->raw_vec = 1;  // FP64 moments, one column per lane
-    pl->nstrips = (p->na + kStripRows - 1) / kStripRows;
+    // Strips of the statistics pass: 128 rows, or fewer (down to 16) while the launch would leave CUs without a
+    // workgroup: each strip re-reads the row above it, and the reduction reads one partial per strip and tile. (ERS block,
+    // 4096 rows: 96 workgroups of 128 rows take 55 us, 768 of 16 rows 27 us.)
+    {
+        int ntiles = 0, nslots = 0;
+        raw_tiles(pl, pl->raw_vec, &ntiles, &nslots);
+        pl->strip_rows = kStripRows;
+        while (pl->strip_rows > 16 && (long)((p->na + pl->strip_rows - 1) / pl->strip_rows) * ntiles < 768) pl->strip_rows /= 2;
+    }
+    pl->nstrips = (p->na + pl->strip_rows - 1) / pl->strip_rows;
     auto fail = [&](int st) {
         plan_free(pl);
         delete pl;
         return st;
     };
     int st = ASARF_OK;
-    pl->rplan = get_plan(c, nrp, kRowThreads, &st);
-    if (!pl->rplan) return fail(st);
+    // the padded line has to have a transform, also where the block kernels do without it
+    {
+        std::vector<int> radices;
+        const auto t = c->tuned_rows.find(nrp);
+        if (!(t != c->tuned_rows.end() && t->second.plan) && !radix_plan_relaxed(nrp, kRowThreads, radices)) {
+            (void)get_plan(c, nrp, kRowThreads, &st);  // sets the error
+            return fail(st);
+        }
+    }
     st = get_col_split(c, nap, &pl->cs);
     if (st != ASARF_OK) return fail(st);
     // ASARF_RCMC_ROW=1: always the row RCMC kernel (the column-tiled kernel is not launched); for comparisons
@@ -235,7 +335,6 @@ extern "C" int asarf_plan_create(asarf_ctx* c, const asarf_focus_params* p, cons
     // second image: the passes ping-pong between the two (A img -> img2, B img2 -> img, RCMC img -> img2,
     // B' img2 -> img, A' img -> img2), since out-of-place passes stream faster than in-place ones
     if ((st = plan_alloc(pl, (void**)&pl->img2, sizeof(float2) * (size_t)nap * pl->stride))) return fail(st);
-    if ((st = plan_alloc(pl, (void**)&pl->hconj, sizeof(float2) * (size_t)nrp))) return fail(st);
     if ((st = plan_alloc(pl, (void**)&pl->col, sizeof(ColConst) * (size_t)nrv))) return fail(st);
     size_t partial_vals = 0;  // the larger of the two tilings (the width is chosen per call from the raw alignment)
     for (int v : {1, pl->raw_vec >= 4 ? 4 : 1, pl->raw_vec}) {
@@ -253,23 +352,6 @@ extern "C" int asarf_plan_create(asarf_ctx* c, const asarf_focus_params* p, cons
         (st = plan_alloc(pl, (void**)&pl->fbaq_lut, sizeof(float2) * 4096)))
         return fail(st);
 
-    // chirp spectrum conj(FFT(chirp))/n: inverse-direction transform of the conjugated chirp
-    {
-        std::vector<float2> h(nrp);
-        for (int i = 0; i < nrp; ++i) h[i] = make_float2(chirp_iq[2 * i], -chirp_iq[2 * i + 1]);
-        if (hipMemcpy(pl->hconj, h.data(), sizeof(float2) * (size_t)nrp, hipMemcpyHostToDevice) != hipSuccess)
-            return fail(set_error(ASARF_EHIP, "asarf_plan_create: chirp upload"));
-        RowFftArgs a{};
-        a.in = pl->hconj;
-        a.in_stride = nrp;
-        a.out = pl->hconj;
-        a.out_stride = nrp;
-        a.rows = 1;
-        a.scale = 1.0f / (float)nrp;
-        a.plan = pl->rplan->dev();
-        if (launch_row_fft(a, true, c->stream) != hipSuccess)
-            return fail(set_error(ASARF_EHIP, "asarf_plan_create: chirp transform"));
-    }
     // Lines are compressed in blocks when the chirp ends within its nc samples and a compiled block length suits
     // (any line length does; see k_rc_block.hip). ASARF_RC_BLOCK=0 keeps the transforms of the padded line,
     // ASARF_RC_BLOCK=<n> takes block length n (comparison runs and tests).
@@ -283,6 +365,8 @@ extern "C" int asarf_plan_create(asarf_ctx* c, const asarf_focus_params* p, cons
     } else {
         pl->rcb = RcBlock{};
     }
+    pl->chirp.assign(chirp_iq, chirp_iq + 2L * nrp);
+    if (padded_lines(pl) && (st = padded_spectrum(pl)) != ASARF_OK) return fail(st);
     // results window (main_flow.cc:155-201) for both signs of the Doppler constant term
     const int max_ap = aperture_pixels_max(p->wavelength, p->prf, p->az_bandwidth_fraction, p->vr_poly,
                                            p->slant_range_first, p->range_spacing, p->nr, p->nc);
@@ -347,6 +431,7 @@ extern "C" int asarf_plan_create(asarf_ctx* c, const asarf_focus_params* p, cons
             (st = plan_alloc(pl, (void**)&pl->ml, sizeof(float) * (size_t)pl->imp_cap * pl->nr_s)))
             return fail(st);
     }
+    pl->core_certain = pl->core && doppler_reach_bound(*p, nblocks, step, nrv) <= kAzCoreReach;
     if (pl->core) {
         // One chunk by default: with the 48-column tiles of the long strided passes (141 KB of LDS) a pass-A'
         // workgroup cannot share a CU with a core workgroup (60 KB), and the two-stream chunks measured slower on
@@ -430,6 +515,7 @@ static int enqueue_to_spectrum(asarf_plan* pl, const void* raw, bool core_path) 
     rm.lines = pl->lines;
     raw_tiles(pl, rm.vec, &rm.ntiles, &rm.nslots);
     rm.nstrips = pl->nstrips;
+    rm.strip_rows = pl->strip_rows;
     rm.partials = pl->partials;
     HIP_CHECK(launch_raw_moments(rm, p.raw_format, s));
     ST_CHECK(mark(pl, "raw_moments"));
@@ -443,6 +529,7 @@ static int enqueue_to_spectrum(asarf_plan* pl, const void* raw, bool core_path) 
     rr.step = pl->step;
     rr.nblocks = pl->nblocks;
     rr.totals = pl->totals;
+    rr.clear = &pl->res->rcmc_reach;
     rr.f64 = p.raw_format == ASARF_RAW_ASAR_FBAQ4;
     HIP_CHECK(launch_reduce_raw(rr, s));
     ST_CHECK(mark(pl, "reduce"));
@@ -463,12 +550,9 @@ static int enqueue_to_spectrum(asarf_plan* pl, const void* raw, bool core_path) 
     fa.imp_in_rows_neg = p.na - pl->crop_neg[0] - pl->crop_neg[1];
     fa.ml_ratio = p.imp ? pl->ml_ratio : 0.f;
     fa.res = pl->res;
-    HIP_CHECK(launch_finalize(fa, s));
-    ST_CHECK(mark(pl, "finalize"));
     ColConstArgs ca{};
     ca.col = pl->col;
     ca.nrv = pl->nrv;
-    ca.dc_poly = pl->res->dc_poly;
     for (int i = 0; i < 3; ++i) ca.vr_poly[i] = p.vr_poly[i];
     ca.wavelength = p.wavelength;
     ca.range_spacing = p.range_spacing;
@@ -476,8 +560,8 @@ static int enqueue_to_spectrum(asarf_plan* pl, const void* raw, bool core_path) 
     ca.prf = p.prf;
     ca.nbins = pl->nap;
     ca.reach = &pl->res->rcmc_reach;
-    HIP_CHECK(launch_col_const(ca, s));
-    ST_CHECK(mark(pl, "column_constants"));
+    HIP_CHECK(launch_finalize(fa, ca, s));
+    ST_CHECK(mark(pl, "finalize"));
     // 2. fused range compression
     RcArgs ra{};
     ra.in = raw;
@@ -490,26 +574,32 @@ static int enqueue_to_spectrum(asarf_plan* pl, const void* raw, bool core_path) 
     ra.zero_to = pl->nrv;
     ra.coef = &pl->res->coef;
     ra.lines = pl->lines;
-    // A saved or measured choice of the autotuner other than the default, or ASARF_RC_VARIANT=<v> (comparison runs
-    // and tests), runs the transforms of the padded line.
-    const auto t = c->tuned_rows.find(pl->nrp);
-    const bool tuned_static = t == c->tuned_rows.end() || t->second.use_static;
-    const int tuned_variant = t == c->tuned_rows.end() ? 0 : t->second.static_variant;
-    const char* v_env = std::getenv("ASARF_RC_VARIANT");
-    const bool forced = v_env && range_compress_static_variants(pl->nrp) > 0;
-    if (pl->rcb.n > 0 && !pl->fft_mfma && !forced && tuned_static && tuned_variant == 0) {
+    bool padded = padded_lines(pl);
+    if (padded && !pl->hconj) {
+        // a choice made since the plan was created; under stream capture nothing can be allocated, and the block
+        // kernels give the same lines
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        HIP_CHECK(hipStreamIsCapturing(s, &cap));
+        if (cap != hipStreamCaptureStatusNone)
+            padded = false;
+        else
+            ST_CHECK(padded_spectrum(pl));
+    }
+    if (!padded) {
         ra.hconj = pl->hblk;
         ra.rc_tw = pl->rc_tw;
         ra.blocks = pl->rcb.blocks;
         ra.block_step = pl->rcb.step;
         HIP_CHECK(launch_rc_block(ra, p.raw_format, pl->rcb.n, s));
     } else {
+        const auto t = c->tuned_rows.find(pl->nrp);
         ra.hconj = pl->hconj;
         ra.plan = pl->rplan->dev();
         ra.mfma = pl->fft_mfma;
-        ra.no_static = tuned_static ? 0 : 1;
-        ra.static_variant = tuned_variant;
-        if (forced) {
+        ra.no_static = (t != c->tuned_rows.end() && !t->second.use_static) ? 1 : 0;
+        ra.static_variant = t != c->tuned_rows.end() ? t->second.static_variant : 0;
+        const char* v_env = std::getenv("ASARF_RC_VARIANT");
+        if (v_env && range_compress_static_variants(pl->nrp) > 0) {
             ra.no_static = 0;
             ra.static_variant = std::atoi(v_env) % range_compress_static_variants(pl->nrp);
         }
@@ -522,6 +612,7 @@ static int enqueue_to_spectrum(asarf_plan* pl, const void* raw, bool core_path) 
         ST_CHECK(col_forward_pass(c, pl->cs, 0, pl->img, pl->stride, p.na, pl->img2, pl->stride, pl->nrv,
                                   pl->fft_mfma));
         ST_CHECK(mark(pl, "azimuth_fft_a"));
+        if (core_path && pl->core_certain) return ASARF_OK;  // the core runs pass B
         ST_CHECK(col_forward_pass(c, pl->cs, 1, pl->img2, pl->stride, pl->nap, pl->img, pl->stride, pl->nrv,
                                   pl->fft_mfma, core_path ? &pl->res->rcmc_reach : nullptr));
         ST_CHECK(mark(pl, "azimuth_fft_b"));
@@ -640,16 +731,19 @@ static int plan_execute(asarf_plan* pl, const void* raw, asarf_image* slc, float
         const int* gate = &pl->res->rcmc_reach;
         // the separate kernels for shift bounds beyond the core's halo first (pass B ran above; RCMC img -> img2,
         // then B' img2 -> img), so that the core chunks below read an untouched pass-A output in img2
-        rc.out = pl->img2;
-        rc.fused_gate = gate;
-        rc.tile_gate = gate;
-        HIP_CHECK(launch_rcmc_tile(rc, s));
-        HIP_CHECK(launch_rcmc_mf(rc, s));
-        ColFftArgs ib = col_args(pl->ctx, pl->img2, pl->stride, pl->img, pl->stride, pl->nrv, cs.n1, cs.n2, 1, n,
-                                 cs.n2, 1, n, cs.full->d_tw, 1.f, cs.p2);
-        ib.fused_gate = gate;
-        HIP_CHECK(launch_col_fft(ib, true, s));
-        ST_CHECK(mark(pl, "azimuth_core_wide"));
+        // (not enqueued where no Doppler estimate can exceed the halo: four launches of about 4.6 us each)
+        if (!pl->core_certain) {
+            rc.out = pl->img2;
+            rc.fused_gate = gate;
+            rc.tile_gate = gate;
+            HIP_CHECK(launch_rcmc_tile(rc, s));
+            HIP_CHECK(launch_rcmc_mf(rc, s));
+            ColFftArgs ib = col_args(pl->ctx, pl->img2, pl->stride, pl->img, pl->stride, pl->nrv, cs.n1, cs.n2, 1, n,
+                                     cs.n2, 1, n, cs.full->d_tw, 1.f, cs.p2);
+            ib.fused_gate = gate;
+            HIP_CHECK(launch_col_fft(ib, true, s));
+            ST_CHECK(mark(pl, "azimuth_core_wide"));
+        }
         AzCoreArgs ac{};
         ac.in = pl->img2;
         ac.out = pl->img;
@@ -662,7 +756,7 @@ static int plan_execute(asarf_plan* pl, const void* raw, asarf_image* slc, float
         ac.beta = p.az_bandwidth_fraction;
         ac.tw2 = cs.p2->d_tw;
         ac.tw_full = cs.full->d_tw;
-        ac.gate = gate;
+        ac.gate = pl->core_certain ? nullptr : gate;
         rcmc_window(ac.window);
         // 4. fused azimuth core (img2 -> img) and 5. inverse pass A' in place (img), 1/Nap, rows < Na, per column
         // chunk. Chunk k's core waits for chunk k - 1's core (on the other stream), so it runs beside chunk
@@ -823,7 +917,7 @@ extern "C" int asarf_plan_results(asarf_plan* pl, asarf_focus_results* r) {
     r->crop_far = pl->far;
     r->imp_rows = pl->p.imp ? d.imp_rows : 0;
     r->rcmc_shift_bound = d.rcmc_reach;
-    const bool fused_ran = core_path_of(pl) && d.rcmc_reach <= kAzCoreReach;
+    const bool fused_ran = core_path_of(pl) && (pl->core_certain || d.rcmc_reach <= kAzCoreReach);
     r->azimuth_core_fused = fused_ran ? 1 : 0;
     return clear_error();
 }
@@ -882,6 +976,7 @@ extern "C" int asarf_plan_set_fft(asarf_plan* pl, int precision) {
         return set_error(ASARF_EUNSUPPORTED,
                          "asarf_plan_set_fft: split-bf16 azimuth passes need a %d = n1 x n2 split into 128/256, got "
                          "%d x %d", pl->nap, pl->cs.n1, pl->cs.n2);
+    ST_CHECK(padded_spectrum(pl));
     pl->fft_mfma = 1;
     return clear_error();
 }
