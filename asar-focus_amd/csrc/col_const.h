@@ -1,6 +1,8 @@
 // FP64 constants of one range column (ColConst) and the bound on the RCMC shift over all columns.
 #pragma once
 
+#include <climits>
+
 #include "kernels.h"
 #include "poly.h"
 
@@ -21,6 +23,27 @@ __device__ __forceinline__ void col_const_store(const ColConstArgs& a, int x, co
         c.dc_off = round(dc / step) * step;
         c.shift_k = a.wavelength * a.wavelength * r0 / (8.0 * vr * vr * a.range_spacing);
         c.inv_ka = a.wavelength * r0 / (2.0 * vr * vr);
+        c.shift_b2 = c.shift_k * step * step;
+        c.turns_b2 = 0.5 * c.inv_ka * step * step;
+        c.m_dc = (int)fmin(fmax(round(dc / step), -1e9), 1e9);
+        // alias_about_dc's comparisons of kb * step with the band limits, as whole bins
+        const double half = 0.5 * a.prf;
+        c.alias_hi = INT_MAX;
+        c.alias_lo = INT_MIN;
+        if (dc < 0.0) {
+            const double lim = half + dc;
+            double k = floor(fmin(fmax(lim / step, -1e9), 1e9));
+            if ((k + 1.0) * step <= lim) k += 1.0;
+            if (k * step > lim) k -= 1.0;
+            c.alias_hi = (int)k;
+        } else if (dc > 0.0) {
+            const double lim = -half + dc;
+            double k = ceil(fmin(fmax(lim / step, -1e9), 1e9));
+            if ((k - 1.0) * step >= lim) k -= 1.0;
+            if (k * step < lim) k += 1.0;
+            c.alias_lo = (int)k;
+        }
+        c.pad = 0;
         a.col[x] = c;
         // The aliased bin frequency stays within prf/2 of the centroid, so |f| <= prf/2 + |dc| bounds the
         // shift of every bin (plus one pixel against rounding).

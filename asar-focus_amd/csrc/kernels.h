@@ -121,6 +121,13 @@ struct ColConst {
     double dc_off;    // bin-quantised centroid [Hz]
     double shift_k;   // RCMC shift in pixels per Hz^2: lambda^2 R0 / (8 Vr^2 dr)
     double inv_ka;    // 1 / azimuth FM rate: lambda R0 / (2 Vr^2)
+    // the same on whole frequency bins kb (kb = f nbins / prf), for the fused azimuth core
+    double shift_b2;  // RCMC shift in pixels per bin^2
+    double turns_b2;  // matched-filter phase in turns: turns_b2 (mc^2 + 2 m_dc kb), mc = bins from the centroid
+    int m_dc;         // bin-quantised centroid
+    int alias_hi;     // bins above it alias down by nbins, bins below alias_lo up (alias_about_dc)
+    int alias_lo;
+    int pad;
 };
 
 struct RowFftArgs {
@@ -213,14 +220,13 @@ struct AzCoreArgs {
     int nrv;
     int nbins;             // n1 * n2
     int n1;
-    int col0;              // first produced column (a multiple of az_core_tile_columns())
-    int ntiles;            // produced tiles, from col0 (the last may end at nrv)
-    int items;             // n1 * ntiles
+    int col0, col1;        // produced columns [col0, col1)
     const ColConst* col;
-    double prf, beta;
+    int half_bins;         // bins further than this from the centroid are outside the azimuth band
     const float2* tw2;     // W_n2^m
     const float2* tw_full; // W_nbins^m
-    const int* gate;       // non-null: do nothing when *gate > kAzCoreReach
+    const int* reach;      // bound on the RCMC shift (DevResults::rcmc_reach): picks the columns per tile
+    int gated;             // do nothing when *reach > kAzCoreReach
     float window[16];      // Blackman window of the RCMC interpolator
 };
 
@@ -374,11 +380,12 @@ hipError_t launch_rcmc_mf(const RcmcArgs& a, hipStream_t s);
 hipError_t launch_rcmc_tile(const RcmcArgs& a, hipStream_t s);
 // Fused azimuth core (k_azcore.hip): LDS bytes of a workgroup, produced columns per tile, the second-pass
 // lengths it is compiled for, the once-per-plan LDS limit, the launch.
-size_t az_core_lds_bytes(int n2, int nbins);
+size_t az_core_lds_bytes(int n2);
 int az_core_tile_columns();
 bool az_core_supported(int n2);
 int az_core_lengths(int* out, int capacity);  // the compiled n2 in order of preference; returns their count
-hipError_t az_core_prepare(int n2, int nbins);
+hipError_t az_core_prepare(int n2);
+int az_core_half_bins(double beta, int nbins);
 hipError_t launch_az_core(const AzCoreArgs& a, int n2, hipStream_t s);
 void rcmc_window(float w[16]);
 hipError_t launch_col_const(const ColConstArgs& a, hipStream_t s);

@@ -312,7 +312,7 @@ extern "C" int asarf_plan_create(asarf_ctx* c, const asarf_focus_params* p, cons
         const size_t half_lds = c->max_lds / 2;
         auto two_per_cu = [&](int n1, int n2) {
             const size_t pass_lds = sizeof(float2) * (size_t)(n1 * 33 + tw_lds_elems(n1) + tw_lds_elems(nap));
-            return pass_lds <= half_lds && az_core_lds_bytes(n2, nap) <= half_lds;
+            return pass_lds <= half_lds && az_core_lds_bytes(n2) <= half_lds;
         };
         for (int round = 0; round < 3 && !pl->core; ++round) {
             for (int i = 0; i < nl; ++i) {
@@ -322,8 +322,8 @@ extern "C" int asarf_plan_create(asarf_ctx* c, const asarf_focus_params* p, cons
                 if (round == 0 && !two_per_cu(nap / n2, n2)) continue;
                 ColSplit alt;
                 if (get_col_split(c, nap, &alt, n2) != ASARF_OK || alt.n2 != n2) continue;
-                if (!az_core_supported(n2) || az_core_lds_bytes(n2, nap) > c->max_lds) continue;
-                if (az_core_prepare(n2, nap) != hipSuccess) continue;
+                if (!az_core_supported(n2) || az_core_lds_bytes(n2) > c->max_lds) continue;
+                if (az_core_prepare(n2) != hipSuccess) continue;
                 pl->cs = alt;
                 pl->core = true;
                 break;
@@ -752,11 +752,11 @@ static int plan_execute(asarf_plan* pl, const void* raw, asarf_image* slc, float
         ac.nbins = pl->nap;
         ac.n1 = cs.n1;
         ac.col = pl->col;
-        ac.prf = p.prf;
-        ac.beta = p.az_bandwidth_fraction;
+        ac.half_bins = az_core_half_bins(p.az_bandwidth_fraction, pl->nap);
         ac.tw2 = cs.p2->d_tw;
         ac.tw_full = cs.full->d_tw;
-        ac.gate = pl->core_certain ? nullptr : gate;
+        ac.reach = gate;
+        ac.gated = pl->core_certain ? 0 : 1;
         rcmc_window(ac.window);
         // 4. fused azimuth core (img2 -> img) and 5. inverse pass A' in place (img), 1/Nap, rows < Na, per column
         // chunk. Chunk k's core waits for chunk k - 1's core (on the other stream), so it runs beside chunk
@@ -778,8 +778,7 @@ static int plan_execute(asarf_plan* pl, const void* raw, asarf_image* slc, float
             const int c0 = t0 * tw, c1 = std::min(t1 * tw, pl->nrv);
             if (k > 0) HIP_CHECK(hipStreamWaitEvent(sk, pl->ev_core[k - 1], 0));
             ac.col0 = c0;
-            ac.ntiles = t1 - t0;
-            ac.items = cs.n1 * ac.ntiles;
+            ac.col1 = c1;
             HIP_CHECK(launch_az_core(ac, cs.n2, sk));
             if (chunks > 1) HIP_CHECK(hipEventRecord(pl->ev_core[k], sk));
             if (chunks == 1) ST_CHECK(mark(pl, "azimuth_core_fused"));
