@@ -786,6 +786,26 @@ int col_inverse_pass(asarf_ctx* c, const ColSplit& cs, int pass, float2* img, lo
 }
 }  // namespace asarf
 
+// Bound on the RCMC shift of a Doppler polynomial over the nrv columns, in the terms of k_col_const: evaluated at the
+// ends of 64 intervals; inside one, a quadratic departs from its chord by at most |a| h^2 / 4.
+static int rda_reach_bound(const asarf_rda_params& p, int nrv) {
+    const int parts = 64;
+    const double h = (double)nrv / parts;
+    double worst = 0.0, d0 = std::fabs(polyval(p.dc_poly, 3, 0.0)), v0 = polyval(p.vr_poly, 3, 0.0);
+    for (int i = 1; i <= parts; ++i) {
+        const double x1 = i * h, d1 = std::fabs(polyval(p.dc_poly, 3, x1)), v1 = polyval(p.vr_poly, 3, x1);
+        const double vr = std::min(v0, v1) - std::fabs(p.vr_poly[0]) * h * h / 4.0;
+        if (!(vr > 0.0)) return 1000000;
+        const double f = 0.5 * p.prf + std::max(d0, d1) + std::fabs(p.dc_poly[0]) * h * h / 4.0;
+        const double r0 = p.slant_range_first + x1 * p.range_spacing;
+        worst = std::max(worst, p.wavelength * p.wavelength * r0 / (8.0 * vr * vr * p.range_spacing) * f * f);
+        d0 = d1;
+        v0 = v1;
+    }
+    worst *= 1.0 + 1e-9;
+    return worst < 1e6 ? (int)std::floor(worst + 0.5) + 1 : 1000000;
+}
+
 extern "C" int asarf_range_doppler(asarf_ctx* c, const asarf_rda_params* p, asarf_image* src, asarf_image* out,
                                    asarf_workspace* ws) {
     if (!c || !p || !out) return set_error(ASARF_EINVAL, "asarf_range_doppler: null argument");
@@ -836,13 +856,51 @@ extern "C" int asarf_range_doppler(asarf_ctx* c, const asarf_rda_params* p, asar
     ca.prf = p->prf;
     ca.nbins = nap;
     ca.reach = d_reach;
-    HIP_CHECK(launch_col_const(ca, c->stream));
     auto* s = static_cast<float2*>(src->data);
     auto* o = static_cast<float2*>(out->data);
     const long so = out->x_stride;
+    // src is consumed (the reference trades it away as the new workspace), so where the strides agree it serves as the
+    // second buffer, and with a shift bound within the fused azimuth core's halo (the Doppler polynomial is known
+    // here) the plan's sequence runs: A s -> o, core o -> s, A' s -> o. (ERS block: 145 us for the core against 260 for
+    // pass B, RCMC + matched filter and pass B'.) ASARF_AZ_FUSED=0 keeps the separate kernels.
+    const char* fz_env = std::getenv("ASARF_AZ_FUSED");
+    const int reach = rda_reach_bound(*p, nrv);
+    if (!(fz_env && fz_env[0] == '0') && cs.n2 > 1 && src->x_stride == out->x_stride && s != o && reach <= kAzCoreReach &&
+        c->tuned_col_n1.find(nap) == c->tuned_col_n1.end() && az_core_split(c, nap, 0, &cs)) {
+        ca.clear_reach = 0;
+        ca.reach = nullptr;
+        HIP_CHECK(launch_col_const(ca, c->stream));
+        ST_CHECK(col_forward_pass(c, cs, 0, s, so, na, o, so, nrv));
+        AzCoreArgs ac{};
+        ac.in = o;
+        ac.out = s;
+        ac.stride = so;
+        ac.nrv = nrv;
+        ac.nbins = nap;
+        ac.n1 = cs.n1;
+        ac.col0 = 0;
+        ac.col1 = nrv;
+        ac.col = col;
+        ac.half_bins = az_core_half_bins(p->az_bandwidth_fraction, nap);
+        ac.tw2 = cs.p2->d_tw;
+        ac.tw_full = cs.full->d_tw;
+        ac.reach_value = reach;
+        rcmc_window(ac.window);
+        HIP_CHECK(launch_az_core(ac, cs.n2, c->stream));
+        ST_CHECK(col_inverse_pass_to(c, cs, 1, s, so, o, so, nrv, na, 1.0f / (float)nap));
+        HIP_CHECK(launch_zero_cols(o, so, out->y_stride, nrv, out->x_stride, c->stream));
+        out->x_size = nrv;
+        out->y_size = na;
+        if (adopt) {
+            ws->data = src->data;
+            ws->bytes = asarf_image_bytes(src);
+            *src = asarf_image{nullptr, 0, 0, 0, 0, ASARF_CF32};
+        }
+        return clear_error();
+    }
+    HIP_CHECK(launch_col_const(ca, c->stream));
     if (cs.n2 > 1 && src->x_stride == out->x_stride && s != o) {
-        // src is consumed (the reference trades it away as the new workspace), so it serves as the second buffer
-        // and every pass runs out of place, as in the fused plan: A s -> o, B o -> s, RCMC + matched filter
+        // every pass out of place through the consumed source: A s -> o, B o -> s, RCMC + matched filter
         // s -> o (column-tiled kernel when the device-side shift bound fits its halo, else the row kernel; both
         // are enqueued and the bound makes exactly one of them work), B' o -> s, A' s -> o
         ST_CHECK(col_forward_pass(c, cs, 0, s, so, na, o, so, nrv));

@@ -109,6 +109,9 @@ int check_cf32(const asarf_image* img, const char* who);
 bool radix_plan(int n, int lanes, std::vector<int>& out);
 bool radix_plan_relaxed(int n, int lanes, std::vector<int>& out);
 bool radix_plan_fits(int n, int lanes, const std::vector<int>& radix);
+// The four-step split of an nap-point column transform whose second pass the fused azimuth core is compiled for
+// (n2_only > 0: only that length); false, *cs untouched, when there is none.
+bool az_core_split(asarf_ctx* c, int nap, int n2_only, ColSplit* cs);
 // Column transform passes of a four-step split (api.cpp); mfma selects the split-bfloat16 kernels.
 int col_forward_pass(asarf_ctx* c, const ColSplit& cs, int pass, const float2* in, long in_stride, int in_rows,
                      float2* img, long stride, int ncols, int mfma = 0, const int* fused_gate = nullptr);

@@ -74,7 +74,7 @@ __global__ __launch_bounds__(kAcThreads) __attribute__((amdgpu_waves_per_eu(core
     static_assert(R0 * R1 == N2, "radices must factor N2");
     constexpr int E = core_elems(R0, R1);
     extern __shared__ float2 lds[];
-    const int reach = *a.reach;
+    const int reach = a.reach ? *a.reach : a.reach_value;
     if (a.gated && reach > kAzCoreReach) return;
     const int width = reach <= kAcNarrowReach ? kAcNarrow : kAcWide;
     const int ntiles = (a.col1 - a.col0 + width - 1) / width;
@@ -316,7 +316,7 @@ hipError_t az_core_prepare(int n2) {
 }
 
 hipError_t launch_az_core(const AzCoreArgs& a, int n2, hipStream_t s) {
-    if (!a.in || !a.out || a.in == a.out || a.n1 <= 0 || a.col1 <= a.col0 || !a.reach) return hipErrorInvalidValue;
+    if (!a.in || !a.out || a.in == a.out || a.n1 <= 0 || a.col1 <= a.col0) return hipErrorInvalidValue;
     // the interpolation skips taps 0 and 15 (sinc16_interior): their window weights must be zero
     if (!(std::fabs(a.window[0]) < 1e-12f && std::fabs(a.window[15]) < 1e-12f)) return hipErrorInvalidValue;
     return core_dispatch(a, n2, false, s);

@@ -226,6 +226,7 @@ struct AzCoreArgs {
     const float2* tw2;     // W_n2^m
     const float2* tw_full; // W_nbins^m
     const int* reach;      // bound on the RCMC shift (DevResults::rcmc_reach): picks the columns per tile
+    int reach_value;       // the bound itself where reach is null
     int gated;             // do nothing when *reach > kAzCoreReach
     float window[16];      // Blackman window of the RCMC interpolator
 };
@@ -376,6 +377,8 @@ hipError_t launch_row_mfma(const RowFftArgs& a, bool inverse, hipStream_t s);
 hipError_t launch_col_mfma(const ColFftArgs& a, bool inverse, hipStream_t s);
 bool launch_col_static(const ColFftArgs& a, bool inverse, hipStream_t s, hipError_t* err);
 bool col_static_length(int n);
+// Column transforms of 2 to 15 points (k_col_small.hip): false for other lengths.
+bool launch_col_small(const ColFftArgs& a, bool inverse, hipStream_t s, hipError_t* err);
 hipError_t launch_rcmc_mf(const RcmcArgs& a, hipStream_t s);
 hipError_t launch_rcmc_tile(const RcmcArgs& a, hipStream_t s);
 // Fused azimuth core (k_azcore.hip): LDS bytes of a workgroup, produced columns per tile, the second-pass
