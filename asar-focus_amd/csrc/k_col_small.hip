@@ -1,0 +1,59 @@
+// Column transforms of 2 to 15 points (the strided first pass of a short azimuth transform, 525 = 5 x 105): one lane per
+// column and group holds the whole transform in registers, so there is no LDS, no barrier and every row access is 256
+// contiguous columns. Bounded by launch and memory latency: 525 x 496 columns take 4.6 us a pass, 20 us with the
+// runtime-radix kernel, whose 16 lanes per column share one 5-point butterfly.
+#include "kernels.h"
+
+namespace asarf {
+
+template <bool INV, int N>
+__global__ __launch_bounds__(256) void k_col_small(ColFftArgs a) {
+    if (a.fused_gate && *a.fused_gate <= kAzCoreReach) return;
+    const int x = blockIdx.x * 256 + threadIdx.x;
+    if (x >= a.ncols) return;
+    for (int g = blockIdx.y; g < a.groups; g += gridDim.y) {  // the same for every lane
+        float2 v[N];
+#pragma unroll
+        for (int m = 0; m < N; ++m) {
+            const long r = (long)g * a.in_g + (long)m * a.in_m;
+            v[m] = r < a.in_rows ? a.in[r * a.in_stride + x] : make_float2(0.f, 0.f);
+        }
+        Dft<N, INV>::run(v);
+#pragma unroll
+        for (int k = 0; k < N; ++k) {
+            const long r = (long)g * a.out_g + (long)k * a.out_m;
+            if (r >= a.out_rows) continue;
+            float2 y = v[k];
+            if (a.tw_full) {
+                const float2 w = a.tw_full[(long)g * k];
+                y = INV ? cmulc(y, w) : cmul(y, w);
+            }
+            a.out[r * a.out_stride + x] = cscale(y, a.scale);
+        }
+    }
+}
+
+template <int N>
+static hipError_t launch_small(const ColFftArgs& a, bool inverse, hipStream_t s) {
+    const dim3 grid((a.ncols + 255) / 256, std::min(a.groups, 65535));
+    if (inverse)
+        hipLaunchKernelGGL((k_col_small<true, N>), grid, dim3(256), 0, s, a);
+    else
+        hipLaunchKernelGGL((k_col_small<false, N>), grid, dim3(256), 0, s, a);
+    return hipGetLastError();
+}
+
+bool launch_col_small(const ColFftArgs& a, bool inverse, hipStream_t s, hipError_t* err) {
+    if (a.ncols < 1 || a.groups < 1) return false;
+    switch (a.sub.n) {
+#define ASARF_COL_SMALL(N) \
+    case N: *err = launch_small<N>(a, inverse, s); return true;
+        ASARF_COL_SMALL(2) ASARF_COL_SMALL(3) ASARF_COL_SMALL(4) ASARF_COL_SMALL(5) ASARF_COL_SMALL(6)
+        ASARF_COL_SMALL(7) ASARF_COL_SMALL(8) ASARF_COL_SMALL(9) ASARF_COL_SMALL(10) ASARF_COL_SMALL(12)
+        ASARF_COL_SMALL(14) ASARF_COL_SMALL(15)
+#undef ASARF_COL_SMALL
+        default: return false;
+    }
+}
+
+}  // namespace asarf

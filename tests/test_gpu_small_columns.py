@@ -1,0 +1,52 @@
+"""Column transforms of 2 to 15 points in registers, and record rows at every pixel remainder and address."""
+import numpy as np
+import pytest
+import torch
+
+import pyoracle as po
+from asarf import _lib as L
+from asarf import focus
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n1", [2, 3, 4, 5, 6, 7, 8, 9, 10, 12, 14, 15])
+@pytest.mark.parametrize("cols", [1, 255, 257])
+def test_short_first_pass(n1, cols, tmp_path):
+    """n1 x 105 column transforms with the split forced through the tuner cache file, against numpy in FP64; an FP32
+    transform of at most 1575 points stays within 2^-24 * sqrt(2 log2 n) * 4 < 1.2e-6 of it."""
+    ctx = focus.Context(0)
+    path = str(tmp_path / "tune.txt")
+    focus.tune_save(ctx, path)
+    n = n1 * 105
+    with open(path, "a") as f:
+        f.write(f"col {n} {n1}\n")
+    focus.tune_load(ctx, path)
+    x = (np.random.default_rng(n).standard_normal((n, cols, 2)) @ [1, 1j]).astype(np.complex64)
+    t = torch.from_numpy(x).cuda()
+    focus.fft(ctx, t, L.FFT_COLUMNS)
+    ref = np.fft.fft(x.astype(np.complex128), axis=0)
+    assert np.linalg.norm(t.cpu().numpy() - ref) < 1.2e-6 * np.linalg.norm(ref)
+    focus.fft(ctx, t, L.FFT_COLUMNS, inverse=True, scale=1.0 / n)
+    assert np.linalg.norm(t.cpu().numpy() - x) < 2.4e-6 * np.linalg.norm(x)
+    ctx.close()
+
+
+@pytest.mark.parametrize("cols", [17, 18, 19, 20, 23, 24, 25, 1023, 1024, 1025])
+@pytest.mark.parametrize("header", [0, 1, 16, 17])
+def test_record_rows(ctx, cols, header):
+    """Whole 16-byte groups and every remainder, equal to the oracle's records byte for byte (detected values away from
+    whole decibels, where single-precision logarithms may differ by an ulp)."""
+    rng = np.random.default_rng(cols + header)
+    v = (rng.standard_normal((5, cols, 2)) @ [2e4, 2e4j]).astype(np.complex64)
+    v[0, :3] = [np.nan, 1e9 - 1e9j, -1e9 + 1j * np.inf]
+    got = focus.condition_slc(ctx, torch.from_numpy(v).cuda(), cols, 5, 0.9, header).cpu().numpy()
+    assert np.array_equal(got, po.condition_slc(v, cols, 5, 0.9, header))
+    d = (10 ** ((rng.integers(-5, 60, (5, cols)) + 0.5) / 10)).astype(np.float32)
+    d[1, :3] = [np.nan, 0.0, np.inf]
+    got = focus.condition_detected(ctx, torch.from_numpy(d).cuda(), 1.0, header).cpu().numpy()
+    assert np.array_equal(got, po.condition_detected(d, 1.0, header))
+    m = np.array(focus.image_statistics(ctx, torch.from_numpy(v[1:].copy()).cuda(), cols, 4))
+    ref = np.array([v[1:].real.mean(dtype=np.float64), v[1:].imag.mean(dtype=np.float64),
+                    v[1:].real.std(dtype=np.float64), v[1:].imag.std(dtype=np.float64)])
+    assert np.allclose(m, ref, rtol=1e-9, atol=1e-6)
