@@ -33,16 +33,26 @@ struct Mom6 {
         sqq = fma(q_, q_, sqq);
         siq = fma(i_, q_, siq);
     }
+    // two adjacent samples a load (16 bytes at the row's own alignment), four loads in flight per lane
+    struct __attribute__((packed, aligned(8))) Pair {
+        float v[4];
+    };
     __device__ __forceinline__ void span(const float2* row, int x0, int x1) {
-        int x = x0 + (int)threadIdx.x;
-        for (; x + 3 * kThreads < x1; x += 4 * kThreads) {
-            const float2 v0 = row[x], v1 = row[x + kThreads], v2 = row[x + 2 * kThreads], v3 = row[x + 3 * kThreads];
-            add(v0);
-            add(v1);
-            add(v2);
-            add(v3);
+        int x = x0 + 2 * (int)threadIdx.x;
+        for (; x + 6 * kThreads + 1 < x1; x += 8 * kThreads) {
+            Pair p[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) p[k] = *reinterpret_cast<const Pair*>(row + x + 2 * k * kThreads);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                add(make_float2(p[k].v[0], p[k].v[1]));
+                add(make_float2(p[k].v[2], p[k].v[3]));
+            }
         }
-        for (; x < x1; x += kThreads) add(row[x]);
+        for (; x < x1; x += 2 * kThreads) {
+            add(row[x]);
+            if (x + 1 < x1) add(row[x + 1]);
+        }
     }
 };
 
@@ -333,7 +343,9 @@ __global__ __launch_bounds__(kThreads) void k_raw_moments(RawMomentsArgs a) {
     }
 }
 
-// Eight columns per lane (one 16-byte load per row: four 32-bit words of two I/Q byte pairs), with the sums of
+// Eight columns per lane (one 16-byte load per row at the row's own alignment: four 32-bit words of two I/Q byte pairs;
+// the lane at the end of a row that is no multiple of eight columns loads the row's last eight and shifts the columns of
+// its neighbour out, so that missing columns are zero bytes; 28411 x 5423: 94 us, 114 with one column a lane), with the sums of
 // squares, cross products and lag-1 products of both pairs of a word in one packed 8-bit dot product each:
 // with mi = w & 0x00FF00FF (the two I bytes) and mq = (w >> 8) & 0x00FF00FF (the two Q bytes),
 // dot4(mi, mi) = I0^2 + I1^2, dot4(mi, mq) = I0 Q0 + I1 Q1, dot4(mi_prev, mq) = I0' Q0 + I1' Q1, ...
@@ -359,9 +371,29 @@ __global__ __launch_bounds__(kThreads) void k_raw_moments8(RawMomentsArgs a) {
     const int x0 = (tile * kThreads + threadIdx.x) * V;
     const int y0 = strip * a.strip_rows;
     const int y1 = min(y0 + a.strip_rows, a.na);
-    const bool valid = x0 < a.nr;  // nr % 8 == 0: all eight columns of the lane, or none
-    const unsigned char* raw = static_cast<const unsigned char*>(a.raw);
-    auto load_row = [&](int y) -> uint4 { return *reinterpret_cast<const uint4*>(raw + ((long)y * a.nr + x0) * 2); };
+    const bool valid = x0 < a.nr;
+    const int cols = min(V, a.nr - x0);  // valid columns of the lane
+    const bool partial = valid && cols < V;
+    const unsigned char* raw = static_cast<const unsigned char*>(a.raw) + 2 * (partial ? a.nr - V : x0);
+    struct __attribute__((packed, aligned(1))) Bytes16 {
+        unsigned w[4];
+    };
+    auto load_row = [&](int y) -> uint4 {
+        const Bytes16 b = *reinterpret_cast<const Bytes16*>(raw + (long)y * a.nr * 2);
+        return make_uint4(b.w[0], b.w[1], b.w[2], b.w[3]);
+    };
+    // a partial lane's row: its columns moved to the front, zero bytes behind them
+    auto front = [&](unsigned (&w)[NW]) {
+        const int drop = V - cols;  // columns of the neighbour
+        for (int i = 0; i < drop >> 1; ++i) {
+#pragma unroll
+            for (int k = 0; k < NW; ++k) w[k] = k + 1 < NW ? w[k + 1] : 0u;
+        }
+        if (drop & 1) {
+#pragma unroll
+            for (int k = 0; k < NW; ++k) w[k] = (w[k] >> 16) | (k + 1 < NW ? w[k + 1] << 16 : 0u);
+        }
+    };
     int sii = 0, sqq = 0, siq = 0;
     int wi[NW], wq[NW], lii[NW], lqq[NW], liq[NW], lqi[NW];
     unsigned pmi[NW], pmq[NW];
@@ -390,7 +422,8 @@ __global__ __launch_bounds__(kThreads) void k_raw_moments8(RawMomentsArgs a) {
     };
     if (valid) {
         const uint4 w = load_row(y0 > 0 ? y0 - 1 : 0);
-        const unsigned ws[NW] = {w.x, w.y, w.z, w.w};
+        unsigned ws[NW] = {w.x, w.y, w.z, w.w};
+        if (partial) front(ws);
         if (sb >= 0) {
             const unsigned e = pick(ws);
             s_prev_i = byte_at(e, 16);
@@ -413,7 +446,8 @@ __global__ __launch_bounds__(kThreads) void k_raw_moments8(RawMomentsArgs a) {
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 if (y + u >= y1) break;
-                const unsigned ws2[NW] = {w8[u].x, w8[u].y, w8[u].z, w8[u].w};
+                unsigned ws2[NW] = {w8[u].x, w8[u].y, w8[u].z, w8[u].w};
+                if (partial) front(ws2);
 #pragma unroll
                 for (int k = 0; k < NW; ++k) {
                     const unsigned mi = ws2[k] & MI, mq = (ws2[k] >> 8) & MI;
@@ -468,7 +502,7 @@ __global__ __launch_bounds__(kThreads) void k_raw_moments8(RawMomentsArgs a) {
     int si = 0, sq = 0;
 #pragma unroll
     for (int k = 0; k < NW; ++k) si += wi[k], sq += wq[k];
-    const long long stv[kRawStats] = {si, sq, sii, sqq, siq, (long long)rows * V};
+    const long long stv[kRawStats] = {si, sq, sii, sqq, siq, (long long)rows * cols};
 #pragma unroll
     for (int i = 0; i < kRawStats; ++i) {
         const long long v = wave_sum<long long>(stv[i]);
@@ -484,7 +518,7 @@ __global__ __launch_bounds__(kThreads) void k_raw_moments8(RawMomentsArgs a) {
         const int li1 = wi[k] - last_i + (y0 > 0 ? edge_i[k] : 0);
         const int lq1 = wq[k] - last_q + (y0 > 0 ? edge_q[k] : 0);
         const int c = threadIdx.x * NW + k;
-        const int vals[kRawLag] = {lii[k], lqq[k], liq[k], lqi[k], li1, lq1, li2, lq2, 2 * lag_rows};
+        const int vals[kRawLag] = {lii[k], lqq[k], liq[k], lqi[k], li1, lq1, li2, lq2, max(0, min(2, cols - 2 * k)) * lag_rows};
 #pragma unroll
         for (int i = 0; i < kRawLag; ++i) shl[i][c] = valid ? vals[i] : 0;
     }
@@ -516,98 +550,116 @@ __global__ __launch_bounds__(kThreads) void k_raw_moments8(RawMomentsArgs a) {
 // values, not integers, so the moments are FP64 sums, formed in a fixed order (each lane over its strip's rows,
 // the wave butterfly, the workgroup's waves, then k_reduce_raw over the strips and tiles) and stored as FP64 bit
 // patterns in the int64 partial slots. One range column per lane. Range samples no record sample lands on are the
-// reference decoder's NaN: skipped by the sums, and a lag-1 pair counts only when both of its samples exist. Each
-// group of 8 rows is decoded in phases (record lengths and shifts, then block ids and code bytes, then the table
-// entries) so that the dependent loads of the 8 rows are in flight together. (Staging the 32 KB table in LDS per
-// workgroup measured slower: 0.46 -> 0.67 ms on the ASAR scene; the 16 entries of a block share one cache line.)
+// reference decoder's NaN: skipped by the sums, and a lag-1 pair counts only when both of its samples exist.
+// Rows are decoded 16 at a time from LDS: the record bytes of the tile's 256 columns (16-byte loads) and the 16 table
+// entries of each quantiser block they touch. Four sub-word gathers per sample from global memory were bound by the
+// vector memory unit: 15000 lines of 5622 samples took 252 us, staged 205 us. (Eight rows decoded ahead of their sums,
+// with the lag sums of single samples from the batch's sums: 269 us, the registers cost more waves than the loads gain.)
+constexpr int kFbaqRows = 16;                              // rows per staged batch
+constexpr int kFbaqBlocks = (kThreads + 62) / 63 + 1;      // quantiser blocks 256 consecutive samples can touch
+union FbaqStage {
+    struct {
+        uint4 bytes[kFbaqRows][4 * kFbaqBlocks];
+        float4 rows[kFbaqRows][8 * kFbaqBlocks];
+    } in;
+    double lag[kRawLag][kThreads];
+};
 __global__ __launch_bounds__(kThreads) void k_raw_moments_fbaq(RawMomentsArgs a) {
-    const float2* lut = a.lines.lut;
+    __shared__ FbaqStage sh;
+    __shared__ int row_s0[kStripRows + 1], row_nb[kStripRows + 1];  // first sample, staged bytes of each row
+    const float4* __restrict__ lut = reinterpret_cast<const float4*>(a.lines.lut);
     const int tile = blockIdx.x;
     const int strip = blockIdx.y;
-    const int x = tile * kThreads + threadIdx.x;
+    const int tid = threadIdx.x;
+    const int x = tile * kThreads + tid;
     const int y0 = strip * a.strip_rows;
     const int y1 = min(y0 + a.strip_rows, a.na);
+    const int yf = max(y0 - 1, 0);  // the row above the strip comes first: the lag of its first row
     const bool col_ok = x < a.nr;
     const unsigned char* base = static_cast<const unsigned char*>(a.raw);
     const LinesDesc L = a.lines;
+    const int cols = min(kThreads, a.nr - tile * kThreads);
+    for (int i = tid; i < y1 - yf; i += kThreads) {
+        const unsigned char* rec = base + (long)(yf + i) * L.line_bytes;
+        const int len = (int)min((long)fbaq4_record_length(rec), L.line_bytes - 2);
+        const int s0 = tile * kThreads - L.shift(yf + i), send = s0 + cols;  // samples [max(s0, 0), send)
+        const int q0 = max(s0, 0) / 63, nq = send > 0 ? (send - 1) / 63 - q0 + 1 : 0;
+        row_s0[i] = s0;
+        row_nb[i] = max(min(64 * nq, len - 64 * q0), 0);
+    }
+    __syncthreads();
     double st[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
     double lg[8] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
     double nvalid = 0.0, npairs = 0.0;
-    float2 prev = make_float2(0.f, 0.f);
+    double pi = 0.0, pq = 0.0;
     bool have_prev = false;
-    if (y0 > 0 && col_ok) {
-        const unsigned char* rec = base + (long)(y0 - 1) * L.line_bytes;
-        have_prev = fbaq4_sample(rec, fbaq4_record_length(rec), L.line_bytes, lut, x - L.shift(y0 - 1), &prev);
-    }
-    constexpr int U = 8;
-    for (int y = y0; y < y1; y += U) {
-        int len[U], sh[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            len[u] = 0;
-            sh[u] = 0;
-            if (y + u < y1) {
-                len[u] = fbaq4_record_length(base + (long)(y + u) * L.line_bytes);
-                sh[u] = L.shift(y + u);
+    for (int yb = yf; yb < y1; yb += kFbaqRows) {
+        const int nrow = min(kFbaqRows, y1 - yb);
+        for (int i = tid; i < nrow * 4 * kFbaqBlocks; i += kThreads) {
+            const int u = i / (4 * kFbaqBlocks), c = i % (4 * kFbaqBlocks);
+            const int nb = row_nb[yb - yf + u];
+            if (16 * c >= nb) continue;
+            const unsigned char* src = base + (long)(yb + u) * L.line_bytes + 2 + 64 * (max(row_s0[yb - yf + u], 0) / 63) + 16 * c;
+            unsigned w[4] = {0, 0, 0, 0};
+            if (16 * c + 16 <= nb) {
+                struct __attribute__((packed, aligned(1))) B {
+                    unsigned v[4];
+                };
+                const B d = *reinterpret_cast<const B*>(src);
+                w[0] = d.v[0], w[1] = d.v[1], w[2] = d.v[2], w[3] = d.v[3];
+            } else {
+                for (int k = 0; k < nb - 16 * c; ++k) w[k >> 2] |= (unsigned)src[k] << (8 * (k & 3));
             }
+            sh.in.bytes[u][c] = make_uint4(w[0], w[1], w[2], w[3]);
         }
-        int bid[U], code[U];
-        bool ok[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int smp = x - sh[u];
-            const int blk = smp >= 0 ? smp / 63 : 0;
-            const int k = 64 * blk + 1 + (smp - 63 * blk);
-            ok[u] = col_ok && y + u < y1 && smp >= 0 && k < len[u] && 2 + (long)k < L.line_bytes;
-            bid[u] = code[u] = 0;
-            if (ok[u]) {
-                const unsigned char* rec = base + (long)(y + u) * L.line_bytes;
-                bid[u] = rec[2 + 64 * blk];
-                code[u] = rec[2 + k];
-            }
+        __syncthreads();
+        for (int i = tid; i < nrow * 8 * kFbaqBlocks; i += kThreads) {
+            const int u = i / (8 * kFbaqBlocks), e = i % (8 * kFbaqBlocks);
+            if (64 * (e >> 3) < row_nb[yb - yf + u])
+                sh.in.rows[u][e] = lut[8 * reinterpret_cast<const unsigned char*>(sh.in.bytes[u])[64 * (e >> 3)] + (e & 7)];
         }
-        float2 v[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            v[u] = make_float2(0.f, 0.f);
-            if (ok[u]) {
-                const int ci = code[u] >> 4, cq = code[u] & 15;
-                const float2* lt = lut + 16 * bid[u];
-                v[u] = make_float2(lt[ci > 7 ? 15 - ci : 8 + ci].x, lt[cq > 7 ? 15 - cq : 8 + cq].y);
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            if (y + u >= y1) break;
-            if (ok[u]) {
-                const double ci = v[u].x, cq = v[u].y;
-                st[0] += ci;
-                st[1] += cq;
-                st[2] += ci * ci;
-                st[3] += cq * cq;
-                st[4] += ci * cq;
-                nvalid += 1.0;
-                if (have_prev) {
-                    const double pi = prev.x, pq = prev.y;
-                    lg[0] += pi * ci;
-                    lg[1] += pq * cq;
-                    lg[2] += pi * cq;
-                    lg[3] += pq * ci;
-                    lg[4] += pi;
-                    lg[5] += pq;
-                    lg[6] += ci;
-                    lg[7] += cq;
-                    npairs += 1.0;
+        __syncthreads();
+#pragma unroll 4
+        for (int u = 0; u < nrow; ++u) {
+            const int s = row_s0[yb - yf + u] + tid;
+            const int q0 = max(row_s0[yb - yf + u], 0) / 63;
+            const int blk = max(s, 0) / 63;
+            const int k = max(s, 0) + blk + 1 - 64 * q0;
+            const bool ok = col_ok && s >= 0 && k < row_nb[yb - yf + u];
+            if (ok) {
+                const int code = reinterpret_cast<const unsigned char*>(sh.in.bytes[u])[k], ci = code >> 4, cq = code & 15;
+                const float2* r = reinterpret_cast<const float2*>(sh.in.rows[u]) + 16 * (blk - q0);
+                const double vi = r[ci > 7 ? 15 - ci : 8 + ci].x, vq = r[cq > 7 ? 15 - cq : 8 + cq].y;
+                if (yb + u >= y0) {
+                    st[0] += vi;
+                    st[1] += vq;
+                    st[2] += vi * vi;
+                    st[3] += vq * vq;
+                    st[4] += vi * vq;
+                    nvalid += 1.0;
+                    if (have_prev) {
+                        lg[0] += pi * vi;
+                        lg[1] += pq * vq;
+                        lg[2] += pi * vq;
+                        lg[3] += pq * vi;
+                        lg[4] += pi;
+                        lg[5] += pq;
+                        lg[6] += vi;
+                        lg[7] += vq;
+                        npairs += 1.0;
+                    }
                 }
+                pi = vi;
+                pq = vq;
             }
-            prev = v[u];
-            have_prev = ok[u];
+            have_prev = ok;
         }
+        __syncthreads();  // the batch is read before the next one (or the lag sums) overwrites it
     }
     const int nval = kRawStats + a.nslots * kRawLag;
     long long* out = a.partials + ((long)strip * a.ntiles + tile) * nval;
     __shared__ double shs[kThreads / 64][kRawStats];
-    __shared__ double shl[kRawLag][kThreads];
+    double (&shl)[kRawLag][kThreads] = sh.lag;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
 #pragma unroll
     for (int i = 0; i < kRawStats; ++i) {
@@ -643,10 +695,8 @@ __global__ __launch_bounds__(kThreads) void k_raw_moments_fbaq(RawMomentsArgs a)
 hipError_t launch_raw_moments(const RawMomentsArgs& a, int fmt, hipStream_t s) {
     const dim3 grid(a.ntiles, a.nstrips);
     if (a.vec == 8) {
-        // 16-byte loads of whole rows of eight pairs, at most one block boundary per lane, the straddle columns
-        // into a.corr
-        if (a.nr % 8 != 0 || (reinterpret_cast<uintptr_t>(a.raw) & 15) != 0 || a.step < 8 || !a.corr ||
-            (fmt != RAW_U8 && fmt != RAW_I8))
+        // rows of at least eight pairs, at most one block boundary per lane, the straddle columns into a.corr
+        if (a.nr < 8 || a.step < 8 || !a.corr || (fmt != RAW_U8 && fmt != RAW_I8))
             return hipErrorInvalidValue;
         if (fmt == RAW_U8)
             hipLaunchKernelGGL(k_raw_moments8<false>, grid, dim3(kThreads), 0, s, a);

@@ -289,9 +289,9 @@ extern "C" int asarf_plan_create(asarf_ctx* c, const asarf_focus_params* p, cons
     pl->stride = (nrv + kColTile - 1) / kColTile * kColTile;
     pl->step = step;
     pl->nblocks = nblocks;
-    // 8 columns per lane when the rows allow 16-byte loads and a lane meets at most one Doppler block boundary,
-    // 4 when they allow 8-byte loads, else 1 (the width of a call also depends on the raw buffer's alignment)
-    pl->raw_vec = (p->nr % 8 == 0 && step >= 8) ? 8 : (p->nr % 4 == 0) ? 4 : 1;
+    // 8 columns per lane where a lane meets at most one Doppler block boundary (any row length and alignment), else 4
+    // when the rows allow 8-byte loads (also of the raw buffer of a call), else 1
+    pl->raw_vec = step >= 8 ? 8 : (p->nr % 4 == 0) ? 4 : 1;
     if (p->raw_format == ASARF_RAW_ERS_LINES)  // lanes of 4 samples valid or NaN together, 8-byte loads
         pl->raw_vec = (p->nr % 4 == 0 && p->samples_per_line % 4 == 0 && p->swst_mult % 4 == 0 &&
                        p->line_bytes % 8 == 0)
@@ -518,7 +518,7 @@ static int enqueue_to_spectrum(asarf_plan* pl, const void* raw, bool core_path) 
     rm.step = pl->step;
     rm.nblocks = pl->nblocks;
     const uintptr_t ra_bits = reinterpret_cast<uintptr_t>(raw);
-    rm.vec = (pl->raw_vec == 8 && (ra_bits & 15) == 0) ? 8 : (pl->raw_vec >= 4 && (ra_bits & 7) == 0) ? 4 : 1;
+    rm.vec = pl->raw_vec == 8 ? 8 : (pl->raw_vec == 4 && (ra_bits & 7) == 0) ? 4 : 1;
     rm.corr = pl->corr;
     rm.lines = pl->lines;
     raw_tiles(pl, rm.vec, &rm.ntiles, &rm.nslots);
