@@ -1,4 +1,4 @@
-"""Column transforms of 2 to 15 points in registers, and record rows at every pixel remainder and address."""
+"""Column transforms of 2 to 30 points in registers, and record rows at every pixel remainder and address."""
 import numpy as np
 import pytest
 import torch
@@ -23,6 +23,28 @@ def test_short_first_pass(n1, cols, tmp_path):
         f.write(f"col {n} {n1}\n")
     focus.tune_load(ctx, path)
     x = (np.random.default_rng(n).standard_normal((n, cols, 2)) @ [1, 1j]).astype(np.complex64)
+    t = torch.from_numpy(x).cuda()
+    focus.fft(ctx, t, L.FFT_COLUMNS)
+    ref = np.fft.fft(x.astype(np.complex128), axis=0)
+    assert np.linalg.norm(t.cpu().numpy() - ref) < 1.2e-6 * np.linalg.norm(ref)
+    focus.fft(ctx, t, L.FFT_COLUMNS, inverse=True, scale=1.0 / n)
+    assert np.linalg.norm(t.cpu().numpy() - x) < 2.4e-6 * np.linalg.norm(x)
+    ctx.close()
+
+
+@pytest.mark.parametrize("n1,n2", [(n, 49) for n in (16, 18, 20, 21, 24, 25, 27, 28, 30)] +
+                         [(98, n) for n in (16, 21, 25, 30)] + [(32, 35)])
+def test_register_lengths_in_both_passes(n1, n2, tmp_path):
+    """16 to 30 points in registers as the strided first pass and as the contiguous second one, and the first lengths
+    past them: against numpy in FP64 with the bound of test_short_first_pass (at most 2940 points)."""
+    ctx = focus.Context(0)
+    path = str(tmp_path / "tune.txt")
+    focus.tune_save(ctx, path)
+    n = n1 * n2
+    with open(path, "a") as f:
+        f.write(f"col {n} {n1}\n")
+    focus.tune_load(ctx, path)
+    x = (np.random.default_rng(n).standard_normal((n, 257, 2)) @ [1, 1j]).astype(np.complex64)
     t = torch.from_numpy(x).cuda()
     focus.fft(ctx, t, L.FFT_COLUMNS)
     ref = np.fft.fft(x.astype(np.complex128), axis=0)
