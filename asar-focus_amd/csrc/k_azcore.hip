@@ -270,10 +270,13 @@ static hipError_t core_launch(const AzCoreArgs& a, size_t lds, bool prepare, hip
 // Second-pass lengths with a compiled core and their radix sequences, in the planner's order of preference (the
 // split of the azimuth FFT takes the first whose first-pass length has a compile-time column kernel). 84, 90, 96
 // and 98 were measured on the production scenes; the others cover the azimuth lengths those four do not divide
-// (powers of two, 3^a 5^b, ...). From 125 on the tile takes more than half a CU's LDS (one workgroup per CU).
+// (powers of two, 3^a 5^b, ...). 63 and 49 come last, for the lengths that none of the others divides: azimuth passes
+// of 3087 = 49 x 63 lines by 4912 columns 278 us with the separate kernels, 203 with the core; of 12005 = 245 x 49
+// 1092 and 818. From 125 on the tile takes more than half a CU's LDS (one workgroup per CU).
 #define ASARF_AZ_CORE_LENGTHS(X)                                                                                  \
     X(84, 12, 7) X(90, 9, 10) X(98, 7, 14) X(96, 8, 12) X(80, 10, 8) X(100, 10, 10) X(72, 9, 8) X(105, 15, 7)     \
-    X(81, 9, 9) X(112, 16, 7) X(64, 8, 8) X(120, 12, 10) X(75, 15, 5) X(126, 14, 9) X(128, 16, 8) X(125, 25, 5)
+    X(81, 9, 9) X(112, 16, 7) X(64, 8, 8) X(120, 12, 10) X(75, 15, 5) X(126, 14, 9) X(128, 16, 8) X(125, 25, 5)   \
+    X(63, 9, 7) X(49, 7, 7)
 
 bool az_core_supported(int n2) {
     switch (n2) {

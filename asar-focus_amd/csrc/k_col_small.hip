@@ -3,8 +3,8 @@
 // every row access is 256 contiguous columns. Bounded by launch and memory latency at the shortest (525 x 496 columns:
 // 4.6 us a pass, 20 us with the runtime-radix kernel, whose 16 lanes per column share one 5-point butterfly) and by
 // memory from 16 points on: pass A of 1512 x 4912 columns 2.8 -> 4.6 TB/s, A' 3.4 -> 5.4; of 2058 lines 3.1 -> 4.8 and
-// 3.8 -> 5.8, before with 16 lanes per column and an LDS exchange between two radices of 3 to 7 (most of a wave's time
-// was that barrier). Both passes, in microseconds, of n x 105 by 4912 columns, LDS kernel -> this one: n = 16 82 -> 60,
+// 3.8 -> 5.8, before with 16 lanes per column and an LDS exchange between two radices of 3 to 7.
+// Both passes, in microseconds, of n x 105 by 4912 columns, LDS kernel -> this one: n = 16 82 -> 60,
 // 21 91 -> 73, 25 95 -> 81, 28 99 -> 91, 30 102 -> 95. The line lies at 30 because a transform of n points takes about
 // 4.6 n registers: 32 points leave three waves per SIMD and take 113 us against 106, 40 points 162 against 160. (A
 // four-wave bound spills from 28 points on: 30 points 101 us, 32 points 130.)

@@ -5,7 +5,7 @@ import torch
 
 import pyoracle as po
 from asarf import _lib as L
-from asarf import focus
+from asarf import configs, focus, scene
 
 pytestmark = pytest.mark.gpu
 
@@ -52,6 +52,26 @@ def test_register_lengths_in_both_passes(n1, n2, tmp_path):
     focus.fft(ctx, t, L.FFT_COLUMNS, inverse=True, scale=1.0 / n)
     assert np.linalg.norm(t.cpu().numpy() - x) < 2.4e-6 * np.linalg.norm(x)
     ctx.close()
+
+
+@pytest.mark.parametrize("na,nap", [(1220, 1225), (1310, 1323), (1708, 1715)])
+def test_core_of_49_and_63(ctx, na, nap, monkeypatch):
+    """Azimuth lengths that only 49 or 63 divides take the fused core: against the separate kernels (FP32 rounding of
+    two orders of the same transforms, 2^-24 * sqrt(2 log2 n) * 4 < 1.2e-6 each) and the oracle's interpolation bound."""
+    cfg = configs.ers_block().scaled(na=na, nr=1500, n_targets_az=2, n_targets_rg=2, tgt_az=(0.4, 0.6))
+    assert focus.padding_size(na) == nap
+    raw, _ = scene.generate(cfg)
+    out = []
+    for fused in ("1", "0"):
+        monkeypatch.setenv("ASARF_AZ_FUSED", fused)
+        plan = focus.Plan(ctx, cfg)
+        plan.execute(torch.from_numpy(raw).cuda())
+        assert bool(plan.results()["azimuth_core_fused"]) == (fused == "1")
+        out.append(plan.slc_tensor().cpu().numpy())
+        plan.close()
+    assert np.linalg.norm(out[0] - out[1]) < 1.2e-6 * np.linalg.norm(out[1])
+    ref, _ = po.focus_slc(scene.raw_to_complex(raw), cfg)
+    assert np.linalg.norm(out[0] - ref) < 1e-4 * np.linalg.norm(ref)
 
 
 @pytest.mark.parametrize("cols", [17, 18, 19, 20, 23, 24, 25, 1023, 1024, 1025])
