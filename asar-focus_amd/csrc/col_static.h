@@ -1,5 +1,5 @@
 // Column transforms with compile-time radix sequences (the kernel template and its launcher). The sub-transform
-// lengths of the four-step azimuth FFT that have such a kernel are every 2^a 3^b 5^c 7^d from 32 to 400, listed
+// lengths of the four-step azimuth FFT that have such a kernel are every 2^a 3^b 5^c 7^d from 16 to 400, listed
 // below with their radix sequences and split over six compilation units (k_col_static*.hip) so they build in
 // parallel. Same workgroup layout and global access as k_col_fft (16 lanes per column, 16, 32 or 48 columns, LDS
 // rows of COLS + 1 elements), but two large radices (composite DFTs in registers) replace three or four
@@ -15,26 +15,23 @@
 #pragma once
 #include "kernels.h"
 
-// 16 to 30: one lane per column (k_col_small.hip)
-#define ASARF_COL_SMALL_LENGTHS(X) X(16) X(18) X(20) X(21) X(24) X(25) X(27) X(28) X(30)
-
 #define ASARF_COL_LENGTHS_0(X) \
-    X(35, 7, 5) X(50, 10, 5) X(81, 9, 9) X(90, 10, 9) X(147, 21, 7) X(168, 12, 14) \
+    X(18, 6, 3) X(20, 5, 4) X(35, 7, 5) X(50, 10, 5) X(81, 9, 9) X(90, 10, 9) X(147, 21, 7) X(168, 12, 14) \
     X(180, 12, 15) X(189, 21, 9) X(240, 16, 15) X(320, 20, 16) X(324, 27, 12) X(343, 7, 7, 7)
 #define ASARF_COL_LENGTHS_1(X) \
-    X(32, 8, 4) X(45, 9, 5) X(48, 8, 6) X(125, 25, 5) X(140, 14, 10) X(144, 12, 12) \
+    X(24, 6, 4) X(25, 5, 5) X(32, 8, 4) X(45, 9, 5) X(48, 8, 6) X(125, 25, 5) X(140, 14, 10) X(144, 12, 12) \
     X(150, 15, 10) X(162, 18, 9) X(224, 16, 14) X(250, 25, 10) X(350, 25, 14) X(384, 24, 16)
 #define ASARF_COL_LENGTHS_2(X) \
-    X(54, 9, 6) X(56, 8, 7) X(70, 10, 7) X(96, 12, 8) X(98, 14, 7) X(105, 15, 7) \
+    X(16, 4, 4) X(30, 6, 5) X(54, 9, 6) X(56, 8, 7) X(70, 10, 7) X(96, 12, 8) X(98, 14, 7) X(105, 15, 7) \
     X(112, 16, 7) X(160, 16, 10) X(175, 25, 7) X(300, 25, 12) X(378, 27, 14) X(400, 25, 16)
 #define ASARF_COL_LENGTHS_3(X) \
     X(36, 6, 6) X(63, 9, 7) X(64, 8, 8) X(80, 10, 8) X(108, 12, 9) X(126, 14, 9) X(128, 16, 8) X(135, 15, 9) \
     X(192, 16, 12) X(280, 20, 14) X(288, 24, 12) X(315, 21, 15) X(392, 28, 14)
 #define ASARF_COL_LENGTHS_4(X) \
-    X(40, 8, 5) X(42, 7, 6) X(60, 10, 6) X(75, 15, 5) X(100, 10, 10) X(196, 14, 14) X(210, 15, 14) \
+    X(21, 7, 3) X(40, 8, 5) X(42, 7, 6) X(60, 10, 6) X(75, 15, 5) X(100, 10, 10) X(196, 14, 14) X(210, 15, 14) \
     X(216, 18, 12) X(243, 27, 9) X(245, 7, 5, 7) X(294, 21, 14) X(360, 15, 24)
 #define ASARF_COL_LENGTHS_5(X) \
-    X(49, 7, 7) X(72, 9, 8) X(84, 12, 7) X(120, 12, 10) X(200, 20, 10) X(225, 15, 15) \
+    X(27, 9, 3) X(28, 7, 4) X(49, 7, 7) X(72, 9, 8) X(84, 12, 7) X(120, 12, 10) X(200, 20, 10) X(225, 15, 15) \
     X(252, 21, 12) X(256, 16, 16) X(270, 27, 10) X(336, 12, 28) X(375, 25, 15)
 
 // case label of a listed length (for switch statements over a list)

@@ -7,7 +7,6 @@ namespace asarf {
 // fits the 16 lanes of a column).
 bool col_static_length(int n) {
     switch (n) {
-        ASARF_COL_SMALL_LENGTHS(ASARF_COL_LABEL)
         ASARF_COL_LENGTHS_0(ASARF_COL_LABEL)
         ASARF_COL_LENGTHS_1(ASARF_COL_LABEL)
         ASARF_COL_LENGTHS_2(ASARF_COL_LABEL)

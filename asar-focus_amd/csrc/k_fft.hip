@@ -314,7 +314,7 @@ __global__ __launch_bounds__(kThreads) void k_col_fft(ColFftArgs a) {
 hipError_t launch_col_fft(const ColFftArgs& a, bool inverse, hipStream_t s) {
     if (a.mfma) return launch_col_mfma(a, inverse, s);
     hipError_t serr = hipSuccess;
-    if (!a.no_static && (launch_col_static(a, inverse, s, &serr) || launch_col_small(a, inverse, s, &serr))) return serr;
+    if (!a.no_static && (launch_col_small(a, inverse, s, &serr) || launch_col_static(a, inverse, s, &serr))) return serr;
     if (a.sub.npass == 0) return hipErrorInvalidValue;  // a length planned for its compile-time kernel only
     const size_t lds = sizeof(float2) * (size_t)(a.sub.n * (kColTile + 1) + tw_lds_elems(a.sub.n));
     if (lds > max_lds_bytes()) return hipErrorInvalidValue;

@@ -377,7 +377,8 @@ hipError_t launch_row_mfma(const RowFftArgs& a, bool inverse, hipStream_t s);
 hipError_t launch_col_mfma(const ColFftArgs& a, bool inverse, hipStream_t s);
 bool launch_col_static(const ColFftArgs& a, bool inverse, hipStream_t s, hipError_t* err);
 bool col_static_length(int n);
-// Column transforms of 2 to 30 points (k_col_small.hip): false for other lengths.
+// Column transforms of 2 to 30 points in registers (k_col_small.hip): false for other lengths, and from 16 points on
+// for launches too small to fill the chip.
 bool launch_col_small(const ColFftArgs& a, bool inverse, hipStream_t s, hipError_t* err);
 hipError_t launch_rcmc_mf(const RcmcArgs& a, hipStream_t s);
 hipError_t launch_rcmc_tile(const RcmcArgs& a, hipStream_t s);

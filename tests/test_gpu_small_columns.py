@@ -54,6 +54,31 @@ def test_register_lengths_in_both_passes(n1, n2, tmp_path):
     ctx.close()
 
 
+@pytest.mark.parametrize("n1", [16, 18, 20, 21, 24, 25, 27, 28, 30])
+def test_register_kernel_takes_launches_that_fill_the_chip(n1, tmp_path):
+    """n1 x 49 on 2817 columns (12 x 49 workgroups: registers) and on the first 257 of them alone (2 x 49: LDS): both
+    within the bound of test_short_first_pass of numpy in FP64, and not the same sums in the same order."""
+    ctx = focus.Context(0)
+    path = str(tmp_path / "tune.txt")
+    focus.tune_save(ctx, path)
+    n = n1 * 49
+    with open(path, "a") as f:
+        f.write(f"col {n} {n1}\n")
+    focus.tune_load(ctx, path)
+    x = (np.random.default_rng(n).standard_normal((n, 2817, 2)) @ [1, 1j]).astype(np.complex64)
+    wide, narrow = torch.from_numpy(x).cuda(), torch.from_numpy(x[:, :257].copy()).cuda()
+    focus.fft(ctx, wide, L.FFT_COLUMNS)
+    focus.fft(ctx, narrow, L.FFT_COLUMNS)
+    ref = np.fft.fft(x.astype(np.complex128), axis=0)
+    got, few = wide.cpu().numpy(), narrow.cpu().numpy()
+    assert np.linalg.norm(got - ref) < 1.2e-6 * np.linalg.norm(ref)
+    assert np.linalg.norm(few - ref[:, :257]) < 1.2e-6 * np.linalg.norm(ref[:, :257])
+    assert not np.array_equal(got[:, :257], few)
+    focus.fft(ctx, wide, L.FFT_COLUMNS, inverse=True, scale=1.0 / n)
+    assert np.linalg.norm(wide.cpu().numpy() - x) < 2.4e-6 * np.linalg.norm(x)
+    ctx.close()
+
+
 @pytest.mark.parametrize("na,nap", [(1220, 1225), (1310, 1323), (1708, 1715)])
 def test_core_of_49_and_63(ctx, na, nap, monkeypatch):
     """Azimuth lengths that only 49 or 63 divides take the fused core: against the separate kernels (FP32 rounding of
