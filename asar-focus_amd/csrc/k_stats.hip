@@ -349,10 +349,11 @@ __global__ __launch_bounds__(kThreads) void k_raw_moments(RawMomentsArgs a) {
 // squares, cross products and lag-1 products of both pairs of a word in one packed 8-bit dot product each:
 // with mi = w & 0x00FF00FF (the two I bytes) and mq = (w >> 8) & 0x00FF00FF (the two Q bytes),
 // dot4(mi, mi) = I0^2 + I1^2, dot4(mi, mq) = I0 Q0 + I1 Q1, dot4(mi_prev, mq) = I0' Q0 + I1' Q1, ...
-// Lag sums are kept per word and filed under the Doppler block of the word's first column; where a block starts
-// at an odd column the word straddles two blocks, and the lane holding that column also sums its lag products
-// alone (corr[strip][block] of the arguments, plain integer products in a branch only such lanes take), which the reduction
-// moves to its own block. The lag-row sums of I and Q follow from the per-word column sums and the rows at the
+// Lag sums are kept per word and filed under the Doppler block of the word's first column; where a block starts, or the
+// last one ends inside the row, at an odd column, the word straddles the two sides, and the lane holding that column
+// also sums its lag products alone (corr[strip][block] of the arguments, with one more entry for the end of the last
+// block; plain integer products in a branch only such lanes take), which the reduction moves to the column's own block,
+// or out of the last one. The lag-row sums of I and Q follow from the per-word column sums and the rows at the
 // strip's edges, so the loop carries nine dot products per word and row.
 template <bool SIGNED>
 __device__ __forceinline__ int dot4(unsigned a, unsigned b, int c) {
@@ -401,13 +402,13 @@ __global__ __launch_bounds__(kThreads) void k_raw_moments8(RawMomentsArgs a) {
     for (int k = 0; k < NW; ++k) wi[k] = wq[k] = lii[k] = lqq[k] = liq[k] = lqi[k] = 0, pmi[k] = pmq[k] = 0;
     int edge_i[NW], edge_q[NW];  // row y0 - 1 (strip > 0) or row 0 (strip 0), per word
     bool have_prev = false;
-    // the lane's block start at an odd column c = sb * step (step >= 8: at most one in the lane's eight columns),
+    // the lane's block boundary at an odd column c = sb * step (step >= 8: at most one in the lane's eight columns),
     // the second column of word sk; its lag sums over the strip's lag rows
     int sb = -1, sk = 0;
     if (valid) {
         const int bb = (x0 + a.step - 1) / a.step;
         const int cs = bb * a.step;
-        if (bb >= 1 && bb < a.nblocks && cs < x0 + V && (cs & 1)) {
+        if (bb >= 1 && bb <= a.nblocks && cs < min(x0 + V, a.nr) && (cs & 1)) {
             sb = bb;
             sk = (cs - x0) >> 1;
         }
@@ -488,7 +489,7 @@ __global__ __launch_bounds__(kThreads) void k_raw_moments8(RawMomentsArgs a) {
     }
     if (sb >= 0) {
         const int sv[kRawLag] = {s_ii, s_qq, s_iq, s_qi, s_pi, s_pq, s_ci, s_cq, s_n};
-        long long* cp = a.corr + ((long)strip * a.nblocks + sb) * kRawLag;
+        long long* cp = a.corr + ((long)strip * (a.nblocks + 1) + sb) * kRawLag;
 #pragma unroll
         for (int i = 0; i < kRawLag; ++i) cp[i] = sv[i];
     }
@@ -771,12 +772,13 @@ __global__ __launch_bounds__(kThreads) void k_reduce_raw(RawReduceArgs a) {
             if (slot >= 0 && slot < a.nslots)
                 acc += val(a.partials[((long)strip * a.ntiles + t) * nval + kRawStats + slot * kRawLag + k]);
         }
-        // eight-column tiling: a column that starts block b at an odd index was filed under block b - 1
+        // eight-column tiling: a column that starts block b at an odd index was filed under block b - 1, also the
+        // column behind the last block
         if (!F64 && a.corr) {
             const bool own = b > 0 && ((b * a.step) & 1);
-            const bool next = b + 1 < a.nblocks && (((b + 1) * a.step) & 1);
+            const bool next = (b + 1) * a.step < a.nr && (((b + 1) * a.step) & 1);
             for (int p = threadIdx.x; p < a.nstrips && (own || next); p += kThreads) {
-                const long base = (long)p * a.nblocks;
+                const long base = (long)p * (a.nblocks + 1);
                 if (own) acc += val(a.corr[(base + b) * kRawLag + k]);
                 if (next) acc -= val(a.corr[(base + b + 1) * kRawLag + k]);
             }

@@ -243,17 +243,17 @@ struct RawMomentsArgs {
     int nstrips;
     int strip_rows;   // rows per strip (<= kStripRows)
     long long* partials; // [strip][tile][kRawStats + nslots*kRawLag]
-    long long* corr;     // vec 8: [nstrips][nblocks][kRawLag] lag sums of the odd block-start columns (written for
-                         // odd starts only)
+    long long* corr;     // vec 8: [nstrips][nblocks + 1][kRawLag] lag sums of the odd columns that start a block or
+                         // follow the last one (written for odd columns inside the row only)
     LinesDesc lines;     // RAW_ERS_LINES, RAW_ASAR_FBAQ4: rows are shifted lines, NaN where no sample lands
 };
 
 struct RawReduceArgs {
     const long long* partials;
-    int nstrips, ntiles, nslots, step, nblocks;
+    int nstrips, ntiles, nslots, step, nblocks, nr;
     int tile_cols;      // 256 * vec
-    const long long* corr;  // vec 8: straddle-column lag sums ([nstrips][nblocks][kRawLag]) to move between
-                            // neighbouring blocks (else null)
+    const long long* corr;  // vec 8: straddle-column lag sums ([nstrips][nblocks + 1][kRawLag]) to move between
+                            // neighbouring blocks or out of the last one (else null)
     long long* totals;  // [kRawStats + nblocks*kRawLag]
     int* clear;         // set to 0 (the RCMC shift bound that k_finalize maximises), or null
     int f64;            // partials and totals hold FP64 sums (bit patterns in the int64 slots): RAW_ASAR_FBAQ4

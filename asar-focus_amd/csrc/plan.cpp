@@ -353,7 +353,7 @@ extern "C" int asarf_plan_create(asarf_ctx* c, const asarf_focus_params* p, cons
     if ((st = plan_alloc(pl, (void**)&pl->partials, sizeof(long long) * partial_vals))) return fail(st);
     if ((st = plan_alloc(pl, (void**)&pl->totals, sizeof(long long) * (size_t)(kRawStats + nblocks * kRawLag))))
         return fail(st);
-    if ((st = plan_alloc(pl, (void**)&pl->corr, sizeof(long long) * (size_t)pl->nstrips * nblocks * kRawLag)))
+    if ((st = plan_alloc(pl, (void**)&pl->corr, sizeof(long long) * (size_t)pl->nstrips * (nblocks + 1) * kRawLag)))
         return fail(st);
     if ((st = plan_alloc(pl, (void**)&pl->res, sizeof(DevResults)))) return fail(st);
     if (p->raw_format == ASARF_RAW_ASAR_FBAQ4 &&
@@ -536,6 +536,7 @@ static int enqueue_to_spectrum(asarf_plan* pl, const void* raw, bool core_path) 
     rr.nslots = rm.nslots;
     rr.step = pl->step;
     rr.nblocks = pl->nblocks;
+    rr.nr = p.nr;
     rr.totals = pl->totals;
     rr.clear = &pl->res->rcmc_reach;
     rr.f64 = p.raw_format == ASARF_RAW_ASAR_FBAQ4;

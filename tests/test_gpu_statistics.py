@@ -50,6 +50,32 @@ def test_strips_and_fit_against_numpy(ctx, na, nr, nc, quirks):
     assert np.max(np.abs(np.polyval(got, x) - np.polyval(ref, x))) < 1e-7
 
 
+@pytest.mark.parametrize("na", [2, 16, 33])
+@pytest.mark.parametrize("nr", [298, 300, 367, 959])
+@pytest.mark.parametrize("fmt", ["i8", "u8"])
+def test_blocks_that_end_on_an_odd_column_inside_the_row(ctx, na, nr, fmt):
+    """Without the extra block the last one can end on an odd column before the row's end (300 columns: 33 blocks of 9
+    end at 297), whose neighbour must not enter its lag sums. The sums are exact integers, so every estimate is the
+    oracle's to FP64 rounding (1e-7 of a PRF of 1.7e3 Hz; one column too many in 9 to 29 moves it by whole Hz)."""
+    step = nr // 32
+    assert (nr // step * step) % 2 == 1 and nr // step * step < nr and step >= 8
+    rng = np.random.default_rng(na * nr)
+    base = configs.asar_scene() if fmt == "i8" else configs.ers_block()
+    cfg = base.scaled(na=na, nr=nr, pulse_len=40.2 / base.fs)
+    v = rng.integers(-100, 100, (na, nr, 2)) if fmt == "i8" else rng.integers(0, 32, (na, nr, 2))
+    raw = v.astype(np.int8 if fmt == "i8" else np.uint8)
+    plan = focus.Plan(ctx, cfg, quirks=0)
+    plan.execute(torch.from_numpy(raw).cuda())
+    res = plan.results()
+    nrp = plan.params.nrp
+    plan.close()
+    img = np.zeros((na, nrp), np.complex128)
+    img[:, :nr] = scene.raw_to_complex(raw)
+    po.iq_correction(img, nr, na, quirks=0)
+    _, _, ref = po.doppler_centroid(img, nr, na, cfg.prf, quirks=0)
+    assert len(ref) == nr // step and np.max(np.abs(np.array(res["block_freq"]) - ref)) < 1e-7
+
+
 @pytest.mark.parametrize("sign", [1, -1])
 def test_worst_doppler_estimates_stay_in_the_core(ctx, sign):
     """Block estimates of +-0.49 PRF in the pattern that drives the fitted polynomial furthest out at the near end:
