@@ -892,11 +892,14 @@ __device__ __forceinline__ void finalize_wave(const FinalizeArgs& f, double* dc3
         c.sin_corr = (float)delta;
         c.inv_cos = (float)(1.0 / cosc);
         c.identity = 0;
+        const double ki = rint(dci), kq = rint(dcq);
+        c.ki = (float)ki;
+        c.kq = (float)kq;
         c.ii = (float)ca;
-        c.i0 = (float)cb;
+        c.i0 = (float)(ca * (ki - dci));
         c.qi = (float)cc;
         c.qq = (float)cd;
-        c.q0 = (float)ce;
+        c.q0 = (float)(cc * (ki - dci) + cd * (kq - dcq));
         r->coef = c;
         r->nblocks = f.nblocks;
         r->dc_poly[0] = poly[0];

@@ -94,11 +94,14 @@ __device__ __forceinline__ void fbaq4_row_decode(const unsigned char* rec, long 
 }
 
 // Affine I/Q correction: I' = (I - dc_i) * inv_gain, Q' = (Q - dc_q - I' * sin_corr) * inv_cos, and the same as one
-// affine map, I' = ii I + i0, Q' = qi I + qq Q + q0 (set by k_finalize in FP64; the block range compression uses it).
+// affine map of the samples less a whole number near their mean, I' = ii (I - ki) + i0, Q' = qi (I - ki) + qq (Q - kq)
+// + q0 (set by k_finalize in FP64; the block range compression uses it). The subtraction is exact for bytes, so the
+// coefficients' rounding acts on the signal and not on its mean: offset bytes (mean 15.5, standard deviation 3 to 6) are
+// corrected to 4.3e-8 RMS of the signal, 8.5e-8 by the form above and 1.5e-7 by an affine map of the bytes themselves.
 struct IqCoef {
     float dc_i, dc_q, inv_gain, sin_corr, inv_cos;
     int identity;
-    float ii, i0, qi, qq, q0;
+    float ki, kq, ii, i0, qi, qq, q0;
 };
 
 // Device-resident results of the fused statistics/Doppler stage.

@@ -133,15 +133,20 @@ __global__ __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(WAVES))) void
     const int row = blockIdx.x / a.blocks;
     const int blk = blockIdx.x - row * a.blocks;
     const int x0 = blk * a.block_step;
-    float ii = 1.f, i0 = 0.f, qi = 0.f, qq = 1.f, q0 = 0.f;  // the affine I/Q correction
+    float ki = 0.f, kq = 0.f, ii = 1.f, i0 = 0.f, qi = 0.f, qq = 1.f, q0 = 0.f;  // the affine I/Q correction
     if (FMT != RAW_CF32 && a.coef) {
+        ki = a.coef->ki;
+        kq = a.coef->kq;
         ii = a.coef->ii;
         i0 = a.coef->i0;
         qi = a.coef->qi;
         qq = a.coef->qq;
         q0 = a.coef->q0;
     }
-    auto correct = [&](float i, float q) { return make_float2(fmaf(ii, i, i0), fmaf(qi, i, fmaf(qq, q, q0))); };
+    auto correct = [&](float i, float q) {
+        const float di = i - ki, dq = q - kq;
+        return make_float2(fmaf(ii, di, i0), fmaf(qi, di, fmaf(qq, dq, q0)));
+    };
     float2 v[E], w[E];
     // ---- the block's samples into the first pass's gather positions, corrected on load
     {

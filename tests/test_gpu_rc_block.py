@@ -7,7 +7,8 @@ import numpy as np
 import pytest
 import torch
 
-from asarf import configs, focus
+import pyoracle as po
+from asarf import configs, focus, scene
 
 pytestmark = pytest.mark.gpu
 
@@ -92,3 +93,26 @@ def test_plan_blocks_against_padded_lines(ctx, nr, nc, fmt):
     for block in [""] + lengths:
         err = rel_rms(_slc(ctx, cfg, block, run, **kw), padded)
         assert err < TOL, (block, err)
+
+
+@pytest.mark.parametrize("mean", [(15.5, 15.5), (60.1, 117.7), (117.3, 60.6), (200.3, 201.9)])
+@pytest.mark.parametrize("fmt", ["u8", "lines", "i8"])
+def test_correction_rounds_the_signal_and_not_its_mean(ctx, mean, fmt):
+    """Weak samples on a large offset, which the affine I/Q correction takes out: the SLC stays within the transforms'
+    rounding of the FP64 oracle (TOL: two transform pairs). A coefficient that rounds on the mean leaves a constant of
+    up to 2^-24 * 200 / 2 = 6e-6 of the signal."""
+    rng = np.random.default_rng(int(mean[0] * 10))
+    na, nr, nc, std = 256, 1500, 300, 2.0
+    base = configs.asar_scene() if fmt == "i8" else configs.ers_block()
+    cfg = base.scaled(na=na, nr=nr, pulse_len=(nc + 0.2) / base.fs)
+    v = np.round(rng.standard_normal((na, nr, 2)) * std + np.array(mean) - (128 if fmt == "i8" else 0))
+    raw = v.astype(np.int8 if fmt == "i8" else np.uint8)
+    plan = focus.Plan(ctx, cfg, lines=(nr, 2 * nr, 1) if fmt == "lines" else None)
+    if fmt == "lines":
+        plan.execute_lines(torch.from_numpy(raw.reshape(na, 2 * nr)).cuda(), torch.full((na,), 7, dtype=torch.int16).cuda(), 7)
+    else:
+        plan.execute(torch.from_numpy(raw).cuda())
+    slc = plan.slc_tensor().cpu().numpy()
+    plan.close()
+    ref, _ = po.focus_slc(scene.raw_to_complex(raw), cfg)
+    assert rel_rms(slc, ref) < TOL
