@@ -371,8 +371,8 @@ bool launch_range_compress_pad(const RcArgs& a, int fmt, int variant, hipStream_
 bool rc_block_choose(int nr, int nc, bool single, RcBlock* out, int only = 0);
 int rc_block_radices(int n, int* radices);
 hipError_t launch_rc_block(const RcArgs& a, int fmt, int n, hipStream_t s);
-// The spectrum conj(FFT_n(chirp)) / n of a chirp of nc samples (device) in the order the kernel's lanes read it: bin
-// j + (2 s + e) m at out[2 (s m + j) + e], m = n / (last radix).
+// The spectrum conj(FFT_n(chirp)) / n of a chirp of nc samples (device), scaled so that the lines keep their amplitude,
+// in the order the kernel's lanes read it: bin j + (2 s + e) m at out[2 (s m + j) + e], m = n / (last radix).
 hipError_t launch_rc_block_spectrum(const float2* chirp, int nc, int n, float2* out, hipStream_t s);
 hipError_t launch_col_fft(const ColFftArgs& a, bool inverse, hipStream_t s);
 hipError_t launch_rc_mfma(const RcArgs& a, int raw_format, hipStream_t s);

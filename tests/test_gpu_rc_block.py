@@ -116,3 +116,24 @@ def test_correction_rounds_the_signal_and_not_its_mean(ctx, mean, fmt):
     plan.close()
     ref, _ = po.focus_slc(scene.raw_to_complex(raw), cfg)
     assert rel_rms(slc, ref) < TOL
+
+
+@pytest.mark.parametrize("nr", [1024, 1536, 2048, 2560, 3072, 4096, 6144])
+def test_lines_keep_their_amplitude(ctx, nr):
+    """Least-squares gain of the compressed lines against FP64, every block length: rounding errors of about 1.8e-7 per
+    sample average to below 1e-9 over 256 lines, so what is left is a common scale, bounded by a third of an FP32
+    rounding (2e-8)."""
+    rng = np.random.default_rng(nr)
+    rows, nc = 256, 400
+    stride = focus.padding_size(nr + nc)
+    t = np.arange(nc) / nc - 0.5
+    chirp = np.zeros(stride, np.complex64)
+    chirp[:nc] = np.exp(1j * np.pi * 0.8 * nc * t * t)
+    x = np.zeros((rows, stride), np.complex64)
+    x[:, :nr] = rng.standard_normal((rows, nr)) + 1j * rng.standard_normal((rows, nr))
+    d = torch.from_numpy(x).cuda()
+    focus.range_compression(ctx, d, nr, rows, chirp, nc)
+    got = d.cpu().numpy()[:, :nr - nc].astype(np.complex128)
+    h = np.conj(np.fft.fft(chirp.astype(np.complex128)))
+    ref = np.fft.ifft(np.fft.fft(x.astype(np.complex128), axis=1) * h, axis=1)[:, :nr - nc]
+    assert abs(np.vdot(ref, got) / np.vdot(ref, ref) - 1) < 2e-8
