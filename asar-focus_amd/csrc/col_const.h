@@ -24,8 +24,12 @@ __device__ __forceinline__ void col_const_store(const ColConstArgs& a, int x, co
         c.shift_k = a.wavelength * a.wavelength * r0 / (8.0 * vr * vr * a.range_spacing);
         c.inv_ka = a.wavelength * r0 / (2.0 * vr * vr);
         c.shift_b2 = c.shift_k * step * step;
-        c.turns_b2 = 0.5 * c.inv_ka * step * step;
-        c.m_dc = (int)fmin(fmax(round(dc / step), -1e9), 1e9);
+        // Undefined statistics (a constant channel) leave no centroid: the fused core, which tests the band on whole
+        // bins, then gets a band about 0 and a phase that is NaN, so that the column is NaN as with the FP64 band test
+        // of the separate kernels, and not zero.
+        const bool known = dc - dc == 0.0;
+        c.turns_b2 = known ? 0.5 * c.inv_ka * step * step : dc - dc;
+        c.m_dc = known ? (int)fmin(fmax(round(dc / step), -1e9), 1e9) : 0;
         // alias_about_dc's comparisons of kb * step with the band limits, as whole bins
         const double half = 0.5 * a.prf;
         c.alias_hi = INT_MAX;

@@ -100,3 +100,28 @@ def test_worst_doppler_estimates_stay_in_the_core(ctx, sign):
     assert "azimuth_core_wide" not in names and "azimuth_fft_b" not in names
     ref, _ = po.focus_slc(scene.raw_to_complex(raw), cfg)
     assert float(np.sqrt(np.sum(np.abs(slc - ref) ** 2) / np.sum(np.abs(ref) ** 2))) < 1e-4
+
+
+@pytest.mark.parametrize("what", ["zeros", "constant", "constant Q"])
+@pytest.mark.parametrize("fmt", ["i8", "u8"])
+def test_undefined_statistics_give_the_same_with_and_without_the_core(ctx, what, fmt, monkeypatch):
+    """A channel without variance leaves the I/Q gain and the centroid undefined (a constant Q alone does so without the
+    reference's padding columns in the sums): NaN in every pixel of the SLC, whether the radar's bound on the shift
+    admits the fused core alone or the separate kernels run."""
+    base = configs.asar_scene() if fmt == "i8" else configs.ers_block()
+    cfg = base.scaled(na=600, nr=1300, pulse_len=200.2 / base.fs)
+    raw = np.zeros((cfg.na, cfg.nr, 2), np.int8 if fmt == "i8" else np.uint8)
+    if what != "zeros":
+        raw[...] = 15
+    if what == "constant Q":
+        raw[..., 0] = np.random.default_rng(1).integers(0, 32, (cfg.na, cfg.nr))
+    for fused in ("1", "0"):
+        monkeypatch.setenv("ASARF_AZ_FUSED", fused)
+        plan = focus.Plan(ctx, cfg, quirks=0 if what == "constant Q" else L.QUIRKS_REFERENCE)
+        plan.set_timing(True)
+        plan.execute(torch.from_numpy(raw).cuda())
+        names = set(plan.kernel_times())
+        slc, res = plan.slc_tensor().cpu().numpy(), plan.results()
+        plan.close()
+        assert ("azimuth_core_fused" in names and "azimuth_core_wide" not in names) == (fused == "1")
+        assert np.isnan(res["dc_poly"]).all() and np.isnan(slc.real).all() and np.isnan(slc.imag).all(), fused
