@@ -865,8 +865,21 @@ extern "C" int asarf_range_doppler(asarf_ctx* c, const asarf_rda_params* p, asar
     // pass B, RCMC + matched filter and pass B'.) ASARF_AZ_FUSED=0 keeps the separate kernels.
     const char* fz_env = std::getenv("ASARF_AZ_FUSED");
     const int reach = rda_reach_bound(*p, nrv);
-    if (!(fz_env && fz_env[0] == '0') && cs.n2 > 1 && src->x_stride == out->x_stride && s != o && reach <= kAzCoreReach &&
-        c->tuned_col_n1.find(nap) == c->tuned_col_n1.end() && az_core_split(c, nap, 0, &cs)) {
+    // The split and its tables are found at the first call of a length whatever its shift, so that no later call, which
+    // may be under stream capture, allocates.
+    const ColSplit* core = nullptr;
+    if (!(fz_env && fz_env[0] == '0') && cs.n2 > 1) {
+        auto it = c->core_splits.find(nap);
+        if (it == c->core_splits.end()) {
+            ColSplit found{};
+            if (!az_core_split(c, nap, 0, &found)) found = ColSplit{};
+            it = c->core_splits.emplace(nap, found).first;
+        }
+        if (it->second.n2 > 1) core = &it->second;
+    }
+    if (core && src->x_stride == out->x_stride && s != o && reach <= kAzCoreReach &&
+        c->tuned_col_n1.find(nap) == c->tuned_col_n1.end()) {
+        cs = *core;
         ca.clear_reach = 0;
         ca.reach = nullptr;
         HIP_CHECK(launch_col_const(ca, c->stream));

@@ -59,6 +59,8 @@ struct asarf_ctx {
     std::map<std::pair<int, int>, std::unique_ptr<asarf::FftPlanHost>> plans;
     std::map<int, float2*> tw_tables;
     std::map<int, float4*> rc_tables;  // per block length: the twiddles of the block range compression's passes
+    // per azimuth length: its fused-core split (az_core_split; n = 0: none), found at the length's first range-Doppler call
+    std::map<int, asarf::ColSplit> core_splits;
     // grow-only scratch
     void* d_scratch = nullptr;
     size_t scratch_bytes = 0;

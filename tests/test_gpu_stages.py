@@ -131,6 +131,45 @@ def test_range_doppler_matches_oracle(ctx, na, nrv, dc, wl):
     assert np.all(got[:, nrv:] == 0)
 
 
+def test_range_doppler_under_capture_after_a_call_on_the_separate_kernels():
+    """A length's first call has a migration beyond the core's halo; a gentle one of the same length is then captured
+    without allocating. Each replay gives the eager result, with eager work between the replays."""
+    stream = torch.cuda.Stream()
+    ctx = focus.Context(0, stream=stream)
+    cfg = configs.ers_block()
+    na, nrv = 1500, 400
+    nap = po.next_fft_size(na)
+    x = np.zeros((nap, nrv + 13), np.complex64)
+    x[:na, :nrv] = rand_c((na, nrv), 5)
+    fresh = cuda(x)
+    gentle, steep = focus.rda_params(cfg, [0, 0, 80.0]), focus.rda_params(cfg, [0, 0, 80.0])
+    steep.wavelength *= 8
+    src, out = fresh.clone(), torch.zeros_like(fresh)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        focus.range_doppler(ctx, steep, src, nrv, na, out=out)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        src.copy_(fresh)
+        focus.range_doppler(ctx, gentle, src, nrv, na, out=out)
+    eager_src, eager = fresh.clone(), torch.zeros_like(fresh)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        focus.range_doppler(ctx, gentle, eager_src, nrv, na, out=eager)
+    torch.cuda.synchronize()
+    for _ in range(3):
+        out.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out[:na, :nrv], eager[:na, :nrv])
+        with torch.cuda.stream(stream):
+            focus.range_doppler(ctx, steep, eager_src, nrv, na, out=src)
+        torch.cuda.synchronize()
+    ctx.close()
+
+
 def test_range_doppler_adopts_and_trades_workspace(ctx):
     """RangeDopplerAlgorithm's buffer trading: out adopts ws, ws receives src's memory."""
     cfg = configs.ers_block()
