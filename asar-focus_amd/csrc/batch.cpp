@@ -77,6 +77,7 @@ extern "C" int asarf_batch_create(asarf_ctx* ctx, int n_streams, asarf_batch** o
         c->tuned_col_n1 = ctx->tuned_col_n1;
         for (const auto& kv : ctx->tuned_rows) {
             asarf_ctx::RowTune rt;
+            rt.padded = kv.second.padded;
             rt.use_static = kv.second.use_static;
             rt.static_variant = kv.second.static_variant;
             if (kv.second.plan) {

@@ -66,10 +66,12 @@ struct asarf_ctx {
     size_t scratch_bytes = 0;
     void* h_pinned = nullptr;
     size_t pinned_bytes = 0;
-    // autotuner choices (asarf_autotune_fft): fastest column split (n1) per column length, and per row length
-    // whether the compile-time range-compression kernel wins and otherwise the fastest runtime radix plan
+    // autotuner choices (asarf_autotune_fft): fastest column split (n1) per column length, and per row length the
+    // fastest range compression of padded lines (a compile-time kernel or a runtime radix plan) and whether it was
+    // faster than the blocks, which otherwise keep the lines that they take
     std::map<int, int> tuned_col_n1;
     struct RowTune {
+        bool padded = false;
         bool use_static = true;
         int static_variant = 0;
         const asarf::FftPlanHost* plan = nullptr;

@@ -194,11 +194,11 @@ static void plan_free(asarf_plan* pl) {
     if (pl->s1) (void)hipStreamDestroy(pl->s1);
 }
 
-// Whether an execution transforms padded lines: without a block length, for split-bfloat16 transforms, for a saved or
-// measured choice of the autotuner other than the default, or with ASARF_RC_VARIANT=<v> (comparison runs and tests).
+// Whether an execution transforms padded lines: without a block length, for split-bfloat16 transforms, where the
+// autotuner measured them faster than the blocks, or with ASARF_RC_VARIANT=<v> (comparison runs and tests).
 static bool padded_lines(const asarf_plan* pl) {
     const auto t = pl->ctx->tuned_rows.find(pl->nrp);
-    const bool tuned = t != pl->ctx->tuned_rows.end() && (!t->second.use_static || t->second.static_variant != 0);
+    const bool tuned = t != pl->ctx->tuned_rows.end() && t->second.padded;
     const bool forced = std::getenv("ASARF_RC_VARIANT") && range_compress_static_variants(pl->nrp) > 0;
     return pl->rcb.n == 0 || pl->fft_mfma || tuned || forced;
 }

@@ -1,8 +1,8 @@
 // Autotuner: measures candidate transform schedules on the device and records the fastest per length in the
 // context, where the planner (get_plan, get_col_split) and the plans created afterwards pick them up.
-//   rows (range compression): the block kernels (the default of every length, recorded as variant 0), the
-//     compile-time variants where the length has them (radix sequences and lanes per line), and runtime-radix plans
-//     with the factors of the length in different orders and groupings;
+//   rows (range compression): of padded lines the compile-time variants where the length has them (radix sequences and
+//     lanes per line) and runtime-radix plans with the factors of the length in different orders and groupings, and
+//     next to the fastest of them the blocks, which plans keep unless the padded lines were faster;
 //   columns (azimuth): every two-pass split n1 x n2 (and the single pass where it fits LDS).
 // Timing: one warm-up launch, then the minimum of `reps` launches bracketed by HIP events.
 #include <algorithm>
@@ -137,10 +137,12 @@ extern "C" int asarf_autotune_fft(asarf_ctx* c, int n, int layout, int batch, in
             plans.push_back(p.get());
             c->plans[std::make_pair(n, -1000 - c->tune_key++)] = std::move(p);
         }
-        // candidate -1: the block kernels; -1 (without them) or -2 .. -nv: the compile-time variants of the length
+        // candidates -1 .. -nv: the compile-time variants of the length; -nv - 1: the blocks
         const float4* rc_tw = block ? get_rc_twiddles(c, rb.n, &st) : nullptr;
-        const int nv = std::max(range_compress_static_variants(n), rc_tw ? 1 : 0);
-        for (int ci = -nv; ci < (int)plans.size(); ++ci) {
+        const int nv = range_compress_static_variants(n);
+        float block_ms = INFINITY;
+        for (int ci = rc_tw ? -nv - 1 : -nv; ci < (int)plans.size(); ++ci) {
+            const bool in_blocks = ci < -nv;
             RcArgs a{};
             a.in = raw;
             a.in_stride = nr_in;
@@ -164,7 +166,7 @@ extern "C" int asarf_autotune_fft(asarf_ctx* c, int n, int layout, int batch, in
             a.plan = pd;
             a.no_static = ci >= 0;
             a.static_variant = ci < 0 ? -1 - ci : 0;
-            if (ci == -1 && rc_tw) {
+            if (in_blocks) {
                 a.in_stride = a.nr_in = blk_nr;
                 a.nrv = a.zero_to = blk_nr - blk_nc;
                 a.rc_tw = rc_tw;
@@ -187,7 +189,9 @@ extern "C" int asarf_autotune_fft(asarf_ctx* c, int n, int layout, int batch, in
                 ms_min = std::min(ms_min, ms);
             }
             ++ncand;
-            if (ms_min < best) {
+            if (in_blocks) {
+                block_ms = ms_min;
+            } else if (ms_min < best) {
                 best = ms_min;
                 best_idx = ci;
                 found = true;
@@ -197,6 +201,7 @@ extern "C" int asarf_autotune_fft(asarf_ctx* c, int n, int layout, int batch, in
         cleanup();
         if (!found) return set_error(ASARF_EUNSUPPORTED, "asarf_autotune_fft: no row candidate ran");
         asarf_ctx::RowTune rt;
+        rt.padded = rc_tw && best < block_ms;
         rt.use_static = best_idx < 0;
         rt.static_variant = best_idx < 0 ? -1 - best_idx : 0;
         rt.plan = best_idx >= 0 ? plans[best_idx] : nullptr;
@@ -267,8 +272,11 @@ extern "C" int asarf_autotune_fft(asarf_ctx* c, int n, int layout, int batch, in
 // ------------------------------------------------------------------------------------------ autotuner cache file
 // Text, one choice per line after a header naming the format version and the device architecture:
 //   asarf-tune 1 <gcnArchName>
-//   row <n> static <variant>          compile-time range-compression variant of length n
-//   row <n> radix <r1> <r2> ...       runtime radix order of length n
+//   row <n> static <variant>          compile-time range-compression variant of padded lines of length n
+//   row <n> radix <r1> <r2> ...       runtime radix order of padded lines of length n
+//   row <n> padded static|radix ...   the same, measured faster than the blocks: plans take it for every line (files
+//                                     written before blocks were measured lack the word; their choices are kept for
+//                                     the lines that run padded)
 //   col <n> <n1>                      column split n = n1 x (n / n1) (n1 = n: single pass)
 // Lines starting with '#' and blank lines are skipped.
 
@@ -297,10 +305,11 @@ extern "C" int asarf_tune_save(asarf_ctx* c, const char* path) {
     bool ok = std::fprintf(f, "asarf-tune 1 %s\n", arch.c_str()) > 0;
     for (const auto& kv : c->tuned_rows) {
         const auto& rt = kv.second;
+        const char* padded = rt.padded ? "padded " : "";
         if (rt.use_static || !rt.plan) {
-            ok = ok && std::fprintf(f, "row %d static %d\n", kv.first, rt.static_variant) > 0;
+            ok = ok && std::fprintf(f, "row %d %sstatic %d\n", kv.first, padded, rt.static_variant) > 0;
         } else {
-            ok = ok && std::fprintf(f, "row %d radix", kv.first) > 0;
+            ok = ok && std::fprintf(f, "row %d %sradix", kv.first, padded) > 0;
             for (int r : rt.plan->radix) ok = ok && std::fprintf(f, " %d", r) > 0;
             ok = ok && std::fprintf(f, "\n") > 0;
         }
@@ -319,6 +328,7 @@ extern "C" int asarf_tune_load(asarf_ctx* c, const char* path, int* n_loaded) {
     // parse everything first (no device call): a malformed file changes nothing in the context
     struct RowEntry {
         int n;
+        bool padded;
         bool is_static;
         int variant;
         std::vector<int> radix;
@@ -362,6 +372,8 @@ extern "C" int asarf_tune_load(asarf_ctx* c, const char* path, int* n_loaded) {
             RowEntry e{};
             if (!next_int(&e.n) || e.n < 2) return bad("row: length");
             const char* kind = strtok_r(nullptr, " \t\r\n", &save);
+            e.padded = kind && std::strcmp(kind, "padded") == 0;
+            if (e.padded) kind = strtok_r(nullptr, " \t\r\n", &save);
             if (kind && std::strcmp(kind, "static") == 0) {
                 e.is_static = true;
                 if (!next_int(&e.variant) || e.variant >= std::max(1, range_compress_static_variants(e.n)))
@@ -402,6 +414,7 @@ extern "C" int asarf_tune_load(asarf_ctx* c, const char* path, int* n_loaded) {
                          file_arch.c_str(), arch.c_str());
     for (const auto& e : rows) {
         asarf_ctx::RowTune rt;
+        rt.padded = e.padded;
         rt.use_static = e.is_static;
         rt.static_variant = e.is_static ? e.variant : 0;
         if (!e.is_static) {

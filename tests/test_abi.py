@@ -154,6 +154,17 @@ def test_tuner_cache_rejects_malformed_files_without_device(tmp_path, text, what
         lib.asarf_ctx_destroy(ctx)
 
 
+@pytest.mark.parametrize("text, what", [
+    ("row 6144 padded\n", "'static' or 'radix'"),
+    ("row 6144 padded fast\n", "'static' or 'radix'"),
+    ("row 6144 padded padded static 0\n", "'static' or 'radix'"),
+    ("row 6144 padded static 99\n", "variant"),
+    ("row 6144 padded radix 8 8 8 8\n", "radix order"),
+])
+def test_tuner_cache_checks_padded_rows(tmp_path, text, what):
+    test_tuner_cache_rejects_malformed_files_without_device(tmp_path, "asarf-tune 1 gfx950\n" + text, what)
+
+
 def test_memory_model_trading_without_device():
     """ReleaseMemory / InitExtPtr semantics (device_padded_image.cuh:49-61,104-111) are pure bookkeeping."""
     lib = L.lib()

@@ -78,6 +78,60 @@ def test_tuner_cache_file_round_trip(tmp_path):
     ctx2.close()
 
 
+def _slc_with(monkeypatch, cfg, traw, rows="", **env):
+    """SLC of a plan in a new context with the given tuner file entries, under the given environment."""
+    ctx = focus.Context(0)
+    for k, v in env.items():
+        monkeypatch.setenv(k, v)
+    if rows:
+        path = rows["dir"] / "tune.txt"
+        focus.tune_save(ctx, str(path))
+        path.write_text(path.read_text() + rows["text"] + "\n")
+        focus.tune_load(ctx, str(path))
+        again = rows["dir"] / "again.txt"
+        focus.tune_save(ctx, str(again))
+        assert rows["text"] in again.read_text().splitlines()
+    plan = focus.Plan(ctx, cfg)
+    plan.execute(traw)
+    slc = plan.slc_tensor().cpu().numpy()
+    plan.close()
+    ctx.close()
+    for k in env:
+        monkeypatch.delenv(k)
+    return slc
+
+
+@pytest.mark.parametrize("choice,env", [("static 3", {"ASARF_RC_VARIANT": "3"}), ("radix 8 8 4 5 5", None)])
+def test_padded_row_choices_displace_blocks_only_when_measured_faster(monkeypatch, tmp_path, choice, env):
+    """A row choice without the mark leaves the blocks their lines and is taken where blocks are off; a marked one
+    replaces them. The same kernels give the same bits."""
+    cfg = configs.ers_block().scaled(na=64, n_targets_az=1, n_targets_rg=1)
+    assert focus.padding_size(cfg.nr + cfg.nc) == 6400
+    traw = torch.from_numpy(scene.generate(cfg)[0]).cuda()
+    blocks = _slc_with(monkeypatch, cfg, traw)
+    plain = {"dir": tmp_path, "text": f"row 6400 {choice}"}
+    marked = {"dir": tmp_path, "text": f"row 6400 padded {choice}"}
+    assert np.array_equal(_slc_with(monkeypatch, cfg, traw, plain), blocks)
+    padded = _slc_with(monkeypatch, cfg, traw, plain, ASARF_RC_BLOCK="0")
+    assert not np.array_equal(padded, blocks) and rel_rms(padded, blocks) < 2e-6
+    assert np.array_equal(_slc_with(monkeypatch, cfg, traw, marked), padded)
+    if env:
+        assert np.array_equal(_slc_with(monkeypatch, cfg, traw, **env), padded)
+
+
+def test_row_tuner_measures_the_padded_default_beside_the_blocks(tmp_path):
+    """The recorded choice is one of the padded candidates, whichever way the blocks compare, and the file says which."""
+    ctx = focus.Context(0)
+    r = focus.autotune(ctx, 6400, columns=False, batch=512)
+    focus.tune_save(ctx, str(tmp_path / "tune.txt"))
+    ctx.close()
+    row = [t for t in (tmp_path / "tune.txt").read_text().splitlines() if t.startswith("row 6400 ")]
+    want = f"static {-1 - r['choice']}" if r["choice"] < 0 else "radix "
+    assert len(row) == 1 and row[0].replace("padded ", "").startswith(f"row 6400 {want}")
+    # six compile-time variants and the blocks, beside at least one radix order
+    assert r["choice"] >= -6 and r["candidates"] >= 8
+
+
 def test_batch_graph_equals_sequential_and_replays(ctx):
     cfgs = configs.batch_blocks(6, na_range=(300, 900))
     cfgs = [c.scaled(nr=min(c.nr, 1500)) for c in cfgs]
