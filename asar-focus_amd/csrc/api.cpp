@@ -335,8 +335,8 @@ int get_col_split(asarf_ctx* c, int n, ColSplit* cs, int n2_max) {
 }
 }  // namespace asarf
 
-extern "C" int asarf_ctx_destroy(asarf_ctx* c) {
-    if (!c) return set_error(ASARF_EINVAL, "asarf_ctx_destroy: null");
+void asarf::ctx_unref(asarf_ctx* c) {
+    if (--c->refs > 0) return;
     if (c->initialized) {
         (void)hipSetDevice(c->device);
         (void)hipStreamSynchronize(c->stream);
@@ -347,6 +347,11 @@ extern "C" int asarf_ctx_destroy(asarf_ctx* c) {
         if (c->own_stream && c->stream) (void)hipStreamDestroy(c->stream);
     }
     delete c;
+}
+
+extern "C" int asarf_ctx_destroy(asarf_ctx* c) {
+    if (!c) return set_error(ASARF_EINVAL, "asarf_ctx_destroy: null");
+    ctx_unref(c);
     return clear_error();
 }
 

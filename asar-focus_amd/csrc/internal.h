@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <map>
 #include <memory>
 #include <string>
@@ -47,6 +48,9 @@ struct ColSplit {
 }  // namespace asarf
 
 struct asarf_ctx {
+    // Plans and networks that use the context, and its owner's own reference. Destroying the context with users left
+    // (a garbage collector finalises a cycle in any order) leaves it to the last of them.
+    std::atomic<int> refs{1};
     int device = 0;
     hipStream_t stream = nullptr;
     bool own_stream = false;
@@ -82,6 +86,7 @@ struct asarf_ctx {
 
 namespace asarf {
 int ctx_init(asarf_ctx* ctx);
+void ctx_unref(asarf_ctx* ctx);
 int ctx_scratch(asarf_ctx* ctx, size_t bytes, void** out);
 int ctx_pinned(asarf_ctx* ctx, size_t bytes, void** out);
 const FftPlanHost* get_plan(asarf_ctx* ctx, int n, int lanes, int* status);

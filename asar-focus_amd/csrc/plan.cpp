@@ -462,15 +462,18 @@ extern "C" int asarf_plan_create(asarf_ctx* c, const asarf_focus_params* p, cons
         }
     }
     if (hipStreamSynchronize(c->stream) != hipSuccess) return fail(set_error(ASARF_EHIP, "asarf_plan_create: sync"));
+    ++c->refs;
     *out = pl;
     return clear_error();
 }
 
 extern "C" int asarf_plan_destroy(asarf_plan* pl) {
     if (!pl) return set_error(ASARF_EINVAL, "asarf_plan_destroy: null");
-    (void)hipStreamSynchronize(pl->ctx->stream);
+    asarf_ctx* c = pl->ctx;
+    (void)hipStreamSynchronize(c->stream);
     plan_free(pl);
     delete pl;
+    ctx_unref(c);
     return clear_error();
 }
 

@@ -81,15 +81,18 @@ extern "C" int asarf_rcmc_net_create(asarf_ctx* c, unsigned long long seed, asar
     for (int i = 0; i < kNetOut * kNetH; ++i) p[kNetOW3 + i] = uni(l3);
     if ((st = upload_params(n, p.data())) != ASARF_OK) return fail(st);
     for (int i = 0; i < 8; ++i) n->window8[i] = blackman_value(i, 8);
+    ++c->refs;
     *out = n;
     return clear_error();
 }
 
 extern "C" int asarf_rcmc_net_destroy(asarf_rcmc_net* n) {
     if (!n) return set_error(ASARF_EINVAL, "asarf_rcmc_net_destroy: null");
-    (void)hipStreamSynchronize(n->ctx->stream);
+    asarf_ctx* c = n->ctx;
+    (void)hipStreamSynchronize(c->stream);
     net_free(n);
     delete n;
+    ctx_unref(c);
     return clear_error();
 }
 

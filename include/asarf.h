@@ -73,6 +73,7 @@ typedef struct asarf_ctx asarf_ctx;
  * to the first call that launches work, so argument validation works on hosts without a GPU.
  * Replaces CudaInit (cuda_util/cuda_device_init.h:26-43). */
 int asarf_ctx_create(int device, void* stream, asarf_ctx** out);
+/* A context with plans or networks left is freed with the last of them. */
 int asarf_ctx_destroy(asarf_ctx* ctx);
 int asarf_sync(asarf_ctx* ctx);
 void* asarf_ctx_stream(asarf_ctx* ctx);

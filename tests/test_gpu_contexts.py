@@ -70,3 +70,24 @@ def test_two_contexts_two_threads_keep_their_own_settings():
     for ctx, plan in made.values():
         plan.close()
         ctx.close()
+
+
+def test_context_outlives_its_destruction_while_plans_use_it():
+    """A plan and a network closed after their context, as the collection of a reference cycle may order it: both still
+    work until then and are freed on the context's own stream."""
+    stream = torch.cuda.Stream()
+    ctx = focus.Context(0, stream=stream)
+    cfg = configs.ers_block().scaled(na=64, nr=600, pulse_len=100.2 / 18.96e6)
+    raw = torch.from_numpy(scene.generate(cfg)[0]).cuda()
+    plan, net = focus.Plan(ctx, cfg), focus.RcmcNet(ctx)
+    torch.cuda.synchronize()
+    plan.execute(raw)
+    torch.cuda.synchronize()
+    before = plan.results()
+    ctx.close()
+    plan.execute(raw)
+    torch.cuda.synchronize()
+    assert plan.results() == before
+    assert np.isfinite(net.params()).all()
+    plan.close()
+    net.close()
