@@ -183,6 +183,19 @@ bool radix_plan_relaxed(int n, int lanes, std::vector<int>& out) {
     return !out.empty();
 }
 
+hipError_t table_upload(asarf_ctx* c, void* dst, const void* src, size_t bytes) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    hipError_t e = hipStreamIsCapturing(c->stream, &cap);
+    if (e != hipSuccess) return e;
+    if (cap == hipStreamCaptureStatusNone) return hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice);
+    hipStream_t aside = nullptr;
+    if ((e = hipStreamCreateWithFlags(&aside, hipStreamNonBlocking)) != hipSuccess) return e;
+    e = hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, aside);
+    const hipError_t es = hipStreamSynchronize(aside);
+    (void)hipStreamDestroy(aside);
+    return e != hipSuccess ? e : es;
+}
+
 float2* get_twiddles(asarf_ctx* c, int n, int* status) {
     auto it = c->tw_tables.find(n);
     if (it != c->tw_tables.end()) return it->second;
@@ -197,7 +210,7 @@ float2* get_twiddles(asarf_ctx* c, int n, int* status) {
         *status = set_error(ASARF_ENOMEM, "twiddle table %d: %s", n, hipGetErrorString(e));
         return nullptr;
     }
-    e = hipMemcpy(d, h.data(), sizeof(float2) * (size_t)n, hipMemcpyHostToDevice);
+    e = table_upload(c, d, h.data(), sizeof(float2) * (size_t)n);
     if (e != hipSuccess) {
         *status = set_error(ASARF_EHIP, "twiddle upload: %s", hipGetErrorString(e));
         return nullptr;

@@ -87,6 +87,8 @@ struct asarf_ctx {
 namespace asarf {
 int ctx_init(asarf_ctx* ctx);
 void ctx_unref(asarf_ctx* ctx);
+// Host memory into a table (device). The context's stream may be under capture, where the plain copy would break it.
+hipError_t table_upload(asarf_ctx* ctx, void* dst, const void* src, size_t bytes);
 int ctx_scratch(asarf_ctx* ctx, size_t bytes, void** out);
 int ctx_pinned(asarf_ctx* ctx, size_t bytes, void** out);
 const FftPlanHost* get_plan(asarf_ctx* ctx, int n, int lanes, int* status);

@@ -204,8 +204,8 @@ static bool padded_lines(const asarf_plan* pl) {
 }
 
 // The padded line's transform and the chirp spectrum conj(FFT(chirp))/nrp (inverse-direction transform of the
-// conjugated chirp), built when first needed.
-static int padded_spectrum(asarf_plan* pl) {
+// conjugated chirp), built on the stream when first needed.
+static int padded_spectrum(asarf_plan* pl, hipStream_t stream) {
     if (pl->hconj) return ASARF_OK;
     const int nrp = pl->nrp;
     int st = ASARF_OK;
@@ -223,8 +223,8 @@ static int padded_spectrum(asarf_plan* pl) {
     a.rows = 1;
     a.scale = 1.0f / (float)nrp;
     a.plan = pl->rplan->dev();
-    if (hipMemcpy(d, h.data(), sizeof(float2) * (size_t)nrp, hipMemcpyHostToDevice) != hipSuccess ||
-        launch_row_fft(a, true, pl->ctx->stream) != hipSuccess) {
+    if (table_upload(pl->ctx, d, h.data(), sizeof(float2) * (size_t)nrp) != hipSuccess ||
+        launch_row_fft(a, true, stream) != hipSuccess) {
         (void)hipFree(d);
         pl->bytes -= sizeof(float2) * (size_t)nrp;
         return set_error(ASARF_EHIP, "asarf_plan: chirp spectrum of %d samples", nrp);
@@ -232,6 +232,29 @@ static int padded_spectrum(asarf_plan* pl) {
     pl->hconj = d;
     std::vector<float>().swap(pl->chirp);
     return ASARF_OK;
+}
+
+// padded_spectrum for an execution, whose stream may be under capture: the spectrum belongs to the plan and not to the
+// graph, so it is then built at once on a stream of its own, with this thread's calls exempt from the capture's checks.
+static int padded_spectrum_now(asarf_plan* pl) {
+    if (pl->hconj) return ASARF_OK;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    HIP_CHECK(hipStreamIsCapturing(pl->ctx->stream, &cap));
+    if (cap == hipStreamCaptureStatusNone) return padded_spectrum(pl, pl->ctx->stream);
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    HIP_CHECK(hipThreadExchangeStreamCaptureMode(&mode));
+    hipStream_t aside = nullptr;
+    int st = ASARF_OK;
+    if (hipStreamCreateWithFlags(&aside, hipStreamNonBlocking) != hipSuccess) {
+        st = set_error(ASARF_EHIP, "asarf_plan: stream for the chirp spectrum");
+    } else {
+        st = padded_spectrum(pl, aside);
+        if (hipStreamSynchronize(aside) != hipSuccess && st == ASARF_OK)
+            st = set_error(ASARF_EHIP, "asarf_plan: chirp spectrum of %d samples", pl->nrp);
+        (void)hipStreamDestroy(aside);
+    }
+    HIP_CHECK(hipThreadExchangeStreamCaptureMode(&mode));
+    return st;
 }
 
 extern "C" int asarf_plan_create(asarf_ctx* c, const asarf_focus_params* p, const float* chirp_iq, asarf_plan** out) {
@@ -374,7 +397,7 @@ extern "C" int asarf_plan_create(asarf_ctx* c, const asarf_focus_params* p, cons
         pl->rcb = RcBlock{};
     }
     pl->chirp.assign(chirp_iq, chirp_iq + 2L * nrp);
-    if (padded_lines(pl) && (st = padded_spectrum(pl)) != ASARF_OK) return fail(st);
+    if (padded_lines(pl) && (st = padded_spectrum(pl, c->stream)) != ASARF_OK) return fail(st);
     // results window (main_flow.cc:155-201) for both signs of the Doppler constant term
     const int max_ap = aperture_pixels_max(p->wavelength, p->prf, p->az_bandwidth_fraction, p->vr_poly,
                                            p->slant_range_first, p->range_spacing, p->nr, p->nc);
@@ -586,17 +609,8 @@ static int enqueue_to_spectrum(asarf_plan* pl, const void* raw, bool core_path) 
     ra.zero_to = pl->nrv;
     ra.coef = &pl->res->coef;
     ra.lines = pl->lines;
-    bool padded = padded_lines(pl);
-    if (padded && !pl->hconj) {
-        // a choice made since the plan was created; under stream capture nothing can be allocated, and the block
-        // kernels give the same lines
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        HIP_CHECK(hipStreamIsCapturing(s, &cap));
-        if (cap != hipStreamCaptureStatusNone)
-            padded = false;
-        else
-            ST_CHECK(padded_spectrum(pl));
-    }
+    const bool padded = padded_lines(pl);
+    if (padded) ST_CHECK(padded_spectrum_now(pl));  // for a choice made since the plan was created
     if (!padded) {
         ra.hconj = pl->hblk;
         ra.rc_tw = pl->rc_tw;
@@ -987,7 +1001,7 @@ extern "C" int asarf_plan_set_fft(asarf_plan* pl, int precision) {
         return set_error(ASARF_EUNSUPPORTED,
                          "asarf_plan_set_fft: split-bf16 azimuth passes need a %d = n1 x n2 split into 128/256, got "
                          "%d x %d", pl->nap, pl->cs.n1, pl->cs.n2);
-    ST_CHECK(padded_spectrum(pl));
+    ST_CHECK(padded_spectrum_now(pl));
     pl->fft_mfma = 1;
     return clear_error();
 }

@@ -119,6 +119,49 @@ def test_padded_row_choices_displace_blocks_only_when_measured_faster(monkeypatc
         assert np.array_equal(_slc_with(monkeypatch, cfg, traw, **env), padded)
 
 
+def test_a_choice_made_after_creation_is_captured(monkeypatch, tmp_path):
+    """A plan whose lines run in blocks, captured right after a padded choice was loaded (or forced): every replay gives
+    that choice's bits, with eager work between the replays."""
+    cfg = configs.ers_block().scaled(na=64, n_targets_az=1, n_targets_rg=1)
+    traw = torch.from_numpy(scene.generate(cfg)[0]).cuda()
+    want = _slc_with(monkeypatch, cfg, traw, ASARF_RC_VARIANT="3")
+    for how in ("file", "environment"):
+        stream = torch.cuda.Stream()
+        ctx = focus.Context(0, stream=stream)
+        plan = focus.Plan(ctx, cfg)
+        torch.cuda.synchronize()
+        with torch.cuda.stream(stream):
+            plan.execute(traw)
+            blocks = plan.slc_tensor()
+        torch.cuda.synchronize()
+        assert not np.array_equal(blocks.cpu().numpy(), want)
+        if how == "file":
+            path = tmp_path / "tune.txt"
+            focus.tune_save(ctx, str(path))
+            path.write_text(path.read_text() + "row 6400 padded static 3\n")
+            focus.tune_load(ctx, str(path))
+        else:
+            monkeypatch.setenv("ASARF_RC_VARIANT", "3")
+        graph = torch.cuda.CUDAGraph()
+        out = torch.zeros_like(blocks)
+        with torch.cuda.graph(graph, stream=stream):
+            img = plan.execute(traw)
+            focus.subset_copy(ctx, img, 0, 0, img.x_size, img.y_size, out)
+        for _ in range(3):
+            out.zero_()
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert np.array_equal(out.cpu().numpy(), want), how
+            with torch.cuda.stream(stream):
+                plan.execute(traw)
+            torch.cuda.synchronize()
+        monkeypatch.delenv("ASARF_RC_VARIANT", raising=False)
+        del graph
+        plan.close()
+        ctx.close()
+
+
 def test_row_tuner_measures_the_padded_default_beside_the_blocks(tmp_path):
     """The recorded choice is one of the padded candidates, whichever way the blocks compare, and the file says which."""
     ctx = focus.Context(0)
