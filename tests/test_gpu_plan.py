@@ -174,6 +174,30 @@ def test_plan_statistics_load_width(ctx, nr, offset):
     assert np.abs(np.polyval(res["dc_poly"], xs) - np.polyval(rres["dc_poly"], xs)).max() < 1e-6
 
 
+@pytest.mark.parametrize("fmt", ["i8", "u8", "lines"])
+@pytest.mark.parametrize("offset", [1, 3])
+def test_plan_raw_samples_at_odd_addresses(ctx, fmt, offset):
+    """Samples anywhere in a product file's bytes: bit for bit the results of the aligned copy."""
+    base = configs.asar_scene() if fmt == "i8" else configs.ers_block()
+    cfg = base.scaled(na=300, nr=1403, n_targets_az=1, n_targets_rg=1, n_targets_random=2)
+    raw, _ = scene.generate(cfg)
+    out = []
+    for off in (0, offset):
+        buf = torch.empty(raw.size + 16, dtype=torch.uint8, device="cuda")
+        traw = buf[off:off + raw.size]
+        traw.copy_(torch.from_numpy(raw.reshape(-1).view(np.uint8)))
+        plan = focus.Plan(ctx, cfg, lines=(cfg.nr, 2 * cfg.nr, 4) if fmt == "lines" else None)
+        if fmt == "lines":
+            swst = torch.full((cfg.na,), 700, dtype=torch.int16, device="cuda")
+            plan.execute_lines(traw.view(cfg.na, 2 * cfg.nr), swst, 700)
+        else:
+            plan.execute(traw)
+        out.append((plan.slc_tensor().cpu().numpy(), plan.results()))
+        plan.close()
+    assert np.isfinite(out[0][0].view(np.float32)).all() and np.array_equal(out[0][0], out[1][0])
+    assert out[0][1]["iq"] == out[1][1]["iq"] and out[0][1]["dc_poly"] == out[1][1]["dc_poly"]
+
+
 @pytest.mark.parametrize("na", [1100, 1120, 2500])
 def test_plan_band_edge_sizes(ctx, na):
     """Azimuth lengths (1120, 1125, 2520) for which 0.8 x nbins / 2 is an integer put bins exactly on the band
@@ -235,3 +259,15 @@ def test_plan_azimuth_chunks_are_bit_identical(ctx, chunks):
     np.testing.assert_array_equal(slc_k, slc_1)
     rows = res_1["imp_rows"]
     np.testing.assert_array_equal(imp_k[:rows], imp_1[:rows])
+
+
+@pytest.mark.parametrize("chunks", ["2", "4", "7"])
+def test_plan_azimuth_chunks_with_wide_shifts_are_bit_identical(ctx, chunks):
+    """Chunks of whole 64-column tiles where the shift bound narrows the core's tiles to 56 columns."""
+    cfg = configs.asar_scene()
+    cfg = cfg.scaled(na=1200, nr=3200, n_targets_random=8, wavelength=cfg.wavelength * 2.2)
+    _, slc_1, res_1, _ = run_plan_env(ctx, cfg, {"ASARF_AZ_CHUNKS": "1"})
+    _, slc_k, res_k, _ = run_plan_env(ctx, cfg, {"ASARF_AZ_CHUNKS": chunks})
+    assert res_1["azimuth_core_fused"] and res_k["azimuth_core_fused"]
+    assert 4 <= res_1["rcmc_shift_bound"] <= 8
+    np.testing.assert_array_equal(slc_k, slc_1)

@@ -131,6 +131,33 @@ def test_range_doppler_matches_oracle(ctx, na, nrv, dc, wl):
     assert np.all(got[:, nrv:] == 0)
 
 
+@pytest.mark.parametrize("wl,dc,reach", [(2.5, 80.0, 5), (1.5, -600.0, 5), (1.5, 700.0, 6), (1.9, 700.0, 8)])
+def test_range_doppler_core_with_wide_shifts(ctx, wl, dc, reach, monkeypatch):
+    """Shift bounds of 4 to 8 columns, which the stage entry point hands the fused core by value (tiles of 56 columns):
+    the oracle's image, and that of the separate kernels in another order of sums."""
+    cfg = configs.ers_block()
+    na, nrv = 1500, 400
+    nap = po.next_fft_size(na)
+    lam = cfg.wavelength * wl
+    f = 0.5 * cfg.prf + abs(dc)
+    bound = lam * lam * (cfg.r_first + nrv * cfg.range_spacing) / (8 * cfg.vr ** 2 * cfg.range_spacing) * f * f
+    assert int(bound + 0.5) + 1 == reach
+    src = np.zeros((nap, nrv + 13), np.complex64)
+    src[:na, :nrv] = rand_c((na, nrv), reach)
+    p = focus.rda_params(cfg, [0.0, 0.0, dc])
+    p.wavelength = lam
+    op = po.rda_params(lam, cfg.range_spacing, cfg.r_first, cfg.prf, cfg.az_bandwidth_fraction, [0.0, 0.0, dc],
+                       cfg.vr_poly)
+    ref = po.range_doppler(src.astype(np.complex128), nrv, na, op)
+    core = focus.range_doppler(ctx, p, cuda(src), nrv, na).cpu().numpy()
+    monkeypatch.setenv("ASARF_AZ_FUSED", "0")
+    separate = focus.range_doppler(ctx, p, cuda(src), nrv, na).cpu().numpy()
+    for got in (core, separate):
+        assert rel_rms(got[:na, :nrv], ref[:na, :nrv]) < 1e-5
+        assert np.all(got[:, nrv:] == 0)
+    assert not np.array_equal(core, separate)
+
+
 def test_range_doppler_under_capture_after_a_call_on_the_separate_kernels():
     """A length's first call has a migration beyond the core's halo; a gentle one of the same length is then captured
     without allocating. Each replay gives the eager result, with eager work between the replays."""
