@@ -11,7 +11,8 @@
 // The bound on the shift comes from the device (ColConst), so every workgroup picks its tile width from it; the grid
 // covers the narrow tiles and the surplus workgroups of the wide ones exit at once.
 //
-// What bounds it: vector issue (95 % busy), about half of it RCMC and matched filter, half the transforms. So that
+// What bounds it: vector issue (an instruction on every SIMD cycle; counted with transcendentals as two, 1.09), about
+// half of it RCMC and matched filter, half the transforms. So that
 // * a transform is 8 lanes per column and all 80 columns run at once on 640 of the 768 lanes. 768: a workgroup's waves
 //   go to the SIMDs in order, so two workgroups of 640 lanes put 6 waves on two SIMDs and 4 on the others (1.02 ms on the
 //   ASAR scene against 0.84 ms); the two waves that only take part in phase 2 change places from workgroup to workgroup;
@@ -20,8 +21,8 @@
 // * the twiddles W_N2^(r j) of both directions are one table of N2 entries in LDS (the inverse reads it transposed), and
 //   the inter-pass twiddles W_N^(k1 n) of the workgroup's k1 are another, instead of powers and two-level lookups;
 // * the band test, the aliasing and the phase work on whole bins: integers and one FP64 product chain per pixel.
-// Together 24 % fewer vector instructions (618 M -> 471 M on the ASAR scene, 30240 = 288 x 105, 5095 columns): 1.02 ->
-// 0.84 ms. A copy of its bytes takes 0.49 ms.
+// Together 17 % fewer vector instructions (617 M -> 510 M on the ASAR scene, 30240 = 288 x 105, 5095 columns): 1.02 ->
+// 0.845 ms between HIP events. A copy of its bytes takes 0.49 ms.
 // Phases:
 //   1. forward transforms of the staged columns, bins left in the tile;
 //   2. RCMC + matched filter: lane (wave w, column c) produces bins w, w + 12, ... of column c (a wave reads
@@ -64,7 +65,8 @@ constexpr int core_elems(int r0, int r1) {
     return a > b ? a : b;
 }
 
-// Waves per SIMD the registers leave room for: two workgroups per CU where their tiles fit.
+// Waves per SIMD asked of the compiler: two workgroups per CU where their tiles fit. (90, 100 and 120 bins meet it by
+// spilling 7, 21 and 21 registers, 20 to 36 bytes a lane; the other lengths do without.)
 constexpr int core_waves(int n2) {
     return (size_t)n2 * (kAcPitch + 2) * sizeof(float2) <= 80 * 1024 ? 2 * kAcWaves / 4 : (kAcWaves + 3) / 4;
 }

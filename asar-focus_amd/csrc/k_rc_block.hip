@@ -4,7 +4,8 @@
 
 namespace asarf {
 
-// Compiled lengths: N, lanes, waves per SIMD the registers leave room for, radices. One list per compilation unit.
+// Compiled lengths: N, lanes, waves per SIMD asked of the compiler, radices. One list per compilation unit. (6144 meets
+// its six waves by spilling 7 registers for cf32 lines, 21 for the other formats; the other lengths do without.)
 #define ASARF_RC_BLOCKS_0(X) X(1024, 64, 4, 16, 16, 4) X(1536, 128, 5, 16, 16, 6) X(2048, 128, 4, 16, 16, 8)
 #define ASARF_RC_BLOCKS_1(X) X(2560, 256, 5, 16, 16, 10) X(3072, 256, 5, 16, 16, 12)
 #define ASARF_RC_BLOCKS_2(X) X(4096, 256, 4, 16, 16, 16) X(6144, 512, 6, 8, 8, 8, 12)

@@ -353,9 +353,10 @@ extern "C" int asarf_plan_create(asarf_ctx* c, const asarf_focus_params* p, cons
     pl->rcmc_row_only = row_env && row_env[0] == '1';
     // Fused azimuth core (pass B + RCMC + matched filter + pass B' in one kernel, k_azcore.hip): the default when
     // the azimuth length splits into n1 x n2 with a compiled second-pass length n2 (a short n2 keeps the
-    // workgroup's n2 x 89 spectrum tile within a workgroup's LDS). ASARF_AZ_FUSED=0 keeps the separate kernels (and
-    // the balanced split). Whether the core or the separate kernels run is decided on the device by the RCMC
-    // shift bound (the core's range halo covers shifts up to kAzCoreReach pixels).
+    // workgroup's spectrum tile of n2 bins by 80 columns within its LDS). ASARF_AZ_FUSED=0 keeps the separate kernels
+    // (and the balanced split). The core's range halo covers shifts up to kAzCoreReach pixels: where the host can
+    // prove that none is larger (core_certain), the core runs alone; elsewhere the device decides between it and the
+    // separate kernels by the shift bound of the estimated Doppler polynomial.
     const char* fz_env = std::getenv("ASARF_AZ_FUSED");
     // ASARF_AZ_CORE_N2=<n2> tries only that second-pass length.
     if (!(fz_env && fz_env[0] == '0') && pl->cs.n2 > 1) {
@@ -384,7 +385,7 @@ extern "C" int asarf_plan_create(asarf_ctx* c, const asarf_focus_params* p, cons
         return fail(st);
 
     // Lines are compressed in blocks when the chirp ends within its nc samples and a compiled block length suits
-    // (any line length does; see k_rc_block.hip). ASARF_RC_BLOCK=0 keeps the transforms of the padded line,
+    // (any line length does; rc_block_choose). ASARF_RC_BLOCK=0 keeps the transforms of the padded line,
     // ASARF_RC_BLOCK=<n> takes block length n (comparison runs and tests).
     const char* rb_env = std::getenv("ASARF_RC_BLOCK");
     if (!(rb_env && rb_env[0] == '0') && chirp_tail_zero(chirp_iq, p->nc, nrp) &&
@@ -529,9 +530,8 @@ static int mark(asarf_plan* pl, const char* name) {
 }
 
 // Statistics, Doppler, column constants, range compression and the forward azimuth transform (both passes):
-// on return pl->img holds the range-Doppler image in permuted bin order.
-// Statistics, range compression and the forward azimuth passes. With core_path, pass B is gated on the RCMC shift
-// bound: it runs only where the fused azimuth core (which includes pass B) will not.
+// on return pl->img holds the range-Doppler image in permuted bin order. With core_path, the fused azimuth core
+// includes pass B, which is enqueued only where the core may not run (core_certain unset), gated on the shift bound.
 static int enqueue_to_spectrum(asarf_plan* pl, const void* raw, bool core_path) {
     asarf_ctx* c = pl->ctx;
     const asarf_focus_params& p = pl->p;

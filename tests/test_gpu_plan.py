@@ -150,10 +150,9 @@ def test_plan_tiled_and_row_rcmc_kernels(ctx, wavelength):
 
 @pytest.mark.parametrize("nr,offset", [(1400, 0), (1400, 8), (1400, 2), (1402, 0), (1404, 0)])
 def test_plan_statistics_load_width(ctx, nr, offset):
-    """The raw statistics pass reads 8 samples per lane with 16-byte loads and packed dot products when
-    nr % 8 == 0 and the raw buffer is 16-byte aligned (nr = 1400: Doppler blocks of 43 columns, so every other
-    block starts inside a 2-sample word), 4 samples with 8-byte loads when only nr % 4 == 0 or 8-byte alignment
-    holds, one sample otherwise: each gives the oracle's I/Q statistics, Doppler centroid and SLC."""
+    """The raw statistics pass reads 8 samples per lane with 16-byte loads and packed dot products at any row length and
+    alignment (nr = 1400: Doppler blocks of 43 columns, so every other block starts inside a 2-sample word; nr = 1402:
+    the row's last lane holds two columns): the oracle's I/Q statistics, Doppler centroid and SLC."""
     cfg = configs.asar_scene().scaled(na=640, nr=nr, n_targets_random=4)
     raw, _ = scene.generate(cfg)
     buf = torch.empty(raw.size + 16, dtype=torch.uint8, device="cuda")
