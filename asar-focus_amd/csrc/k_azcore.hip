@@ -11,7 +11,7 @@
 // The bound on the shift comes from the device (ColConst), so every workgroup picks its tile width from it; the grid
 // covers the narrow tiles and the surplus workgroups of the wide ones exit at once.
 //
-// What bounds it: vector issue (an instruction on every SIMD cycle; counted with transcendentals as two, 1.09), about
+// What bounds it: vector issue (an instruction on every SIMD cycle; counted with transcendentals as two, 1.1), about
 // half of it RCMC and matched filter, half the transforms. So that
 // * a transform is 8 lanes per column and all 80 columns run at once on 640 of the 768 lanes. 768: a workgroup's waves
 //   go to the SIMDs in order, so two workgroups of 640 lanes put 6 waves on two SIMDs and 4 on the others (1.02 ms on the
@@ -22,7 +22,7 @@
 //   the inter-pass twiddles W_N^(k1 n) of the workgroup's k1 are another, instead of powers and two-level lookups;
 // * the band test, the aliasing and the phase work on whole bins: integers and one FP64 product chain per pixel.
 // Together 17 % fewer vector instructions (617 M -> 510 M on the ASAR scene, 30240 = 288 x 105, 5095 columns): 1.02 ->
-// 0.845 ms between HIP events. A copy of its bytes takes 0.49 ms.
+// 0.85 ms (0.85 to 0.89 from one card to the next). A copy of its bytes takes 0.49 ms.
 // Phases:
 //   1. forward transforms of the staged columns, bins left in the tile;
 //   2. RCMC + matched filter: lane (wave w, column c) produces bins w, w + 12, ... of column c (a wave reads

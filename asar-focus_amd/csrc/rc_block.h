@@ -9,8 +9,8 @@
 //   N = 256 X (X = 4 .. 16): radices 16, 16, X on 64 to 256 lanes, one to four butterflies per lane and pass
 //   6144: radices 8, 8, 8, 12 on 512 lanes, for lines in place that no shorter length holds
 //
-// What bounds it: vector issue (0.91 of the SIMD cycles; 30000 lines of 5616 samples in 0.54 ms, the padded transforms
-// it replaces 0.64). Per sample and direction three passes cost about 30 FP32 instructions of butterflies and 7.5 of
+// What bounds it: vector issue (0.9 of the SIMD cycles; 30000 lines of 5616 samples in 0.54 to 0.55 ms, the padded
+// transforms it replaces 0.64). Per sample and direction three passes cost about 30 FP32 instructions of butterflies and 7.5 of
 // twiddle products; the rest is kept off the vector units. The samples are loaded straight into the first pass's registers (no
 // staging through LDS, any row alignment). The twiddles of every pass come from a table in global memory (8 to 48 KB,
 // held by L1 and L2) instead of being multiplied up from one power, two a 16-byte load: with 8-byte loads the return
