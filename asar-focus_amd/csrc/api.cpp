@@ -228,16 +228,24 @@ const float4* get_rc_twiddles(asarf_ctx* c, int n, int* status) {
         *status = set_error(ASARF_EUNSUPPORTED, "no block range compression of length %d", n);
         return nullptr;
     }
-    std::vector<float2> h;
+    // the n-th roots of unity from those of the first quadrant (n is a multiple of 4)
+    std::vector<float2> w(n), h;
+    const int q = n / 4;
+    for (int m = 0; m < q; ++m) {
+        const double a = 2.0 * M_PI * (double)m / (double)n;
+        const float x = (float)std::cos(a), y = (float)-std::sin(a);
+        w[m] = make_float2(x, y);
+        w[m + q] = make_float2(y, -x);
+        w[m + 2 * q] = make_float2(-x, -y);
+        w[m + 3 * q] = make_float2(-y, x);
+    }
+    h.reserve((size_t)n + n / 2);
     int ns = radix[0];
     for (int p = 1; p < np; ++p) {
         const int r = radix[p];
-        for (int q = 0; q < r; q += 2)  // pairs of exponents
+        for (int p0 = 0; p0 < r; p0 += 2)  // pairs of exponents
             for (int k = 0; k < ns; ++k)
-                for (int e = q; e < q + 2; ++e) {
-                    const double a = -2.0 * M_PI * (double)((long)e * k) / (double)((long)ns * r);
-                    h.push_back(make_float2((float)std::cos(a), (float)std::sin(a)));
-                }
+                for (int e = p0; e < p0 + 2; ++e) h.push_back(w[(size_t)e * k * (n / (ns * r))]);
         ns *= r;
     }
     float4* d = nullptr;
@@ -278,6 +286,15 @@ const FftPlanHost* get_plan(asarf_ctx* c, int n, int lanes, int* status) {
     const FftPlanHost* raw = p.get();
     c->plans[key] = std::move(p);
     return raw;
+}
+
+int row_transform_exists(asarf_ctx* c, int n) {
+    const auto t = c->tuned_rows.find(n);
+    std::vector<int> radices;
+    if ((t != c->tuned_rows.end() && t->second.plan) || radix_plan_relaxed(n, kRowThreads, radices)) return ASARF_OK;
+    int st = ASARF_OK;
+    (void)get_plan(c, n, kRowThreads, &st);  // sets the error
+    return st;
 }
 
 int get_col_split(asarf_ctx* c, int n, ColSplit* cs, int n2_max) {
@@ -664,9 +681,8 @@ extern "C" int asarf_range_compression(asarf_ctx* c, asarf_image* img, const flo
     if (nc <= 0 || nc >= img->x_size)
         return set_error(ASARF_EINVAL, "asarf_range_compression: chirp samples %d vs range size %d", nc, img->x_size);
     ST_CHECK(ctx_init(c));
-    int st = ASARF_OK;
-    const FftPlanHost* p = get_plan(c, n_chirp, kRowThreads, &st);  // lengths without a transform stay refused
-    if (!p) return st;
+    // the padded line has to have a transform, also where the block kernel does without its tables
+    ST_CHECK(row_transform_exists(c, n_chirp));
     RcArgs a{};
     a.in = img->data;
     a.in_stride = img->x_stride;
@@ -681,6 +697,7 @@ extern "C" int asarf_range_compression(asarf_ctx* c, asarf_image* img, const flo
     RcBlock rb{};
     const bool block = chirp_tail_zero(chirp_iq, nc, n_chirp) && rc_block_choose(img->x_size, nc, true, &rb);
     const int n = block ? rb.n : n_chirp;
+    int st = ASARF_OK;
     void* scratch = nullptr;
     ST_CHECK(ctx_scratch(c, sizeof(float2) * (size_t)n * 2, &scratch));
     float2* d_h = static_cast<float2*>(scratch);
@@ -694,6 +711,8 @@ extern "C" int asarf_range_compression(asarf_ctx* c, asarf_image* img, const flo
         if (!a.rc_tw) return st;
         HIP_CHECK(launch_rc_block(a, RAW_CF32, n, c->stream));
     } else {
+        const FftPlanHost* p = get_plan(c, n_chirp, kRowThreads, &st);
+        if (!p) return st;
         a.nr_in = img->x_stride;
         a.plan = p->dev();
         HIP_CHECK(launch_range_compress(a, RAW_CF32, c->stream));

@@ -92,6 +92,8 @@ hipError_t table_upload(asarf_ctx* ctx, void* dst, const void* src, size_t bytes
 int ctx_scratch(asarf_ctx* ctx, size_t bytes, void** out);
 int ctx_pinned(asarf_ctx* ctx, size_t bytes, void** out);
 const FftPlanHost* get_plan(asarf_ctx* ctx, int n, int lanes, int* status);
+// ASARF_OK where get_plan has a row transform of length n (nothing is built), else its error.
+int row_transform_exists(asarf_ctx* ctx, int n);
 float2* get_twiddles(asarf_ctx* ctx, int n, int* status);
 // Block range compression (rc_block.h): the pass twiddles of block length n.
 const float4* get_rc_twiddles(asarf_ctx* ctx, int n, int* status);

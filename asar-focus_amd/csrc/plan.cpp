@@ -338,14 +338,7 @@ extern "C" int asarf_plan_create(asarf_ctx* c, const asarf_focus_params* p, cons
     };
     int st = ASARF_OK;
     // the padded line has to have a transform, also where the block kernels do without it
-    {
-        std::vector<int> radices;
-        const auto t = c->tuned_rows.find(nrp);
-        if (!(t != c->tuned_rows.end() && t->second.plan) && !radix_plan_relaxed(nrp, kRowThreads, radices)) {
-            (void)get_plan(c, nrp, kRowThreads, &st);  // sets the error
-            return fail(st);
-        }
-    }
+    if ((st = row_transform_exists(c, nrp)) != ASARF_OK) return fail(st);
     st = get_col_split(c, nap, &pl->cs);
     if (st != ASARF_OK) return fail(st);
     // ASARF_RCMC_ROW=1: always the row RCMC kernel (the column-tiled kernel is not launched); for comparisons
