@@ -196,14 +196,29 @@ hipError_t table_upload(asarf_ctx* c, void* dst, const void* src, size_t bytes) 
     return e != hipSuccess ? e : es;
 }
 
+// exp(-2 pi i m / n), m < n, from the values of one quadrant, or of half the circle where n is no multiple of 4.
+static std::vector<float2> roots_of_unity(int n) {
+    std::vector<float2> w(n);
+    const int q = n % 4 == 0 ? n / 4 : 0;
+    for (int m = 0; m < (q ? q : n / 2 + 1); ++m) {
+        const double a = 2.0 * M_PI * (double)m / (double)n;
+        const float x = (float)std::cos(a), y = (float)-std::sin(a);
+        w[m] = make_float2(x, y);
+        if (q) {
+            w[m + q] = make_float2(y, -x);
+            w[m + 2 * q] = make_float2(-x, -y);
+            w[m + 3 * q] = make_float2(-y, x);
+        } else if (m > 0) {
+            w[n - m] = make_float2(x, -y);
+        }
+    }
+    return w;
+}
+
 float2* get_twiddles(asarf_ctx* c, int n, int* status) {
     auto it = c->tw_tables.find(n);
     if (it != c->tw_tables.end()) return it->second;
-    std::vector<float2> h(n);
-    for (int m = 0; m < n; ++m) {
-        const double a = -2.0 * M_PI * (double)m / (double)n;
-        h[m] = make_float2((float)std::cos(a), (float)std::sin(a));
-    }
+    const std::vector<float2> h = roots_of_unity(n);
     float2* d = nullptr;
     hipError_t e = hipMalloc(&d, sizeof(float2) * (size_t)n);
     if (e != hipSuccess) {
@@ -228,17 +243,8 @@ const float4* get_rc_twiddles(asarf_ctx* c, int n, int* status) {
         *status = set_error(ASARF_EUNSUPPORTED, "no block range compression of length %d", n);
         return nullptr;
     }
-    // the n-th roots of unity from those of the first quadrant (n is a multiple of 4)
-    std::vector<float2> w(n), h;
-    const int q = n / 4;
-    for (int m = 0; m < q; ++m) {
-        const double a = 2.0 * M_PI * (double)m / (double)n;
-        const float x = (float)std::cos(a), y = (float)-std::sin(a);
-        w[m] = make_float2(x, y);
-        w[m + q] = make_float2(y, -x);
-        w[m + 2 * q] = make_float2(-x, -y);
-        w[m + 3 * q] = make_float2(-y, x);
-    }
+    const std::vector<float2> w = roots_of_unity(n);
+    std::vector<float2> h;
     h.reserve((size_t)n + n / 2);
     int ns = radix[0];
     for (int p = 1; p < np; ++p) {
@@ -902,20 +908,22 @@ extern "C" int asarf_range_doppler(asarf_ctx* c, const asarf_rda_params* p, asar
     // pass B, RCMC + matched filter and pass B'.) ASARF_AZ_FUSED=0 keeps the separate kernels.
     const char* fz_env = std::getenv("ASARF_AZ_FUSED");
     const int reach = rda_reach_bound(*p, nrv);
-    // The split and its tables are found at the first call of a length whatever its shift, so that no later call, which
-    // may be under stream capture, allocates.
+    // The first such call of a length builds the split's tables, which may be under stream capture after calls beyond the
+    // halo.
     const ColSplit* core = nullptr;
-    if (!(fz_env && fz_env[0] == '0') && cs.n2 > 1) {
+    if (!(fz_env && fz_env[0] == '0') && cs.n2 > 1 && src->x_stride == out->x_stride && s != o && reach <= kAzCoreReach &&
+        c->tuned_col_n1.find(nap) == c->tuned_col_n1.end()) {
         auto it = c->core_splits.find(nap);
         if (it == c->core_splits.end()) {
+            const CaptureExempt exempt(c->stream);
+            HIP_CHECK(exempt.err);
             ColSplit found{};
             if (!az_core_split(c, nap, 0, &found)) found = ColSplit{};
             it = c->core_splits.emplace(nap, found).first;
         }
         if (it->second.n2 > 1) core = &it->second;
     }
-    if (core && src->x_stride == out->x_stride && s != o && reach <= kAzCoreReach &&
-        c->tuned_col_n1.find(nap) == c->tuned_col_n1.end()) {
+    if (core) {
         cs = *core;
         ca.clear_reach = 0;
         ca.reach = nullptr;

@@ -63,7 +63,7 @@ struct asarf_ctx {
     std::map<std::pair<int, int>, std::unique_ptr<asarf::FftPlanHost>> plans;
     std::map<int, float2*> tw_tables;
     std::map<int, float4*> rc_tables;  // per block length: the twiddles of the block range compression's passes
-    // per azimuth length: its fused-core split (az_core_split; n = 0: none), found at the length's first range-Doppler call
+    // per azimuth length: its fused-core split (az_core_split; n = 0: none), found at the first call that asks for it
     std::map<int, asarf::ColSplit> core_splits;
     // grow-only scratch
     void* d_scratch = nullptr;
@@ -87,6 +87,23 @@ struct asarf_ctx {
 namespace asarf {
 int ctx_init(asarf_ctx* ctx);
 void ctx_unref(asarf_ctx* ctx);
+// While it lives, this thread may allocate although the stream is under capture: for tables that belong to a plan or a
+// context and not to the graph.
+struct CaptureExempt {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    hipError_t err;
+    explicit CaptureExempt(hipStream_t s) {
+        err = hipStreamIsCapturing(s, &status);
+        if (err == hipSuccess && capturing()) err = hipThreadExchangeStreamCaptureMode(&mode);
+    }
+    ~CaptureExempt() {
+        if (err == hipSuccess && capturing()) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    }
+    CaptureExempt(const CaptureExempt&) = delete;
+    CaptureExempt& operator=(const CaptureExempt&) = delete;
+    bool capturing() const { return status != hipStreamCaptureStatusNone; }
+};
 // Host memory into a table (device). The context's stream may be under capture, where the plain copy would break it.
 hipError_t table_upload(asarf_ctx* ctx, void* dst, const void* src, size_t bytes);
 int ctx_scratch(asarf_ctx* ctx, size_t bytes, void** out);

@@ -235,25 +235,18 @@ static int padded_spectrum(asarf_plan* pl, hipStream_t stream) {
 }
 
 // padded_spectrum for an execution, whose stream may be under capture: the spectrum belongs to the plan and not to the
-// graph, so it is then built at once on a stream of its own, with this thread's calls exempt from the capture's checks.
+// graph, so it is then built at once on a stream of its own.
 static int padded_spectrum_now(asarf_plan* pl) {
     if (pl->hconj) return ASARF_OK;
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    HIP_CHECK(hipStreamIsCapturing(pl->ctx->stream, &cap));
-    if (cap == hipStreamCaptureStatusNone) return padded_spectrum(pl, pl->ctx->stream);
-    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-    HIP_CHECK(hipThreadExchangeStreamCaptureMode(&mode));
+    const CaptureExempt exempt(pl->ctx->stream);
+    HIP_CHECK(exempt.err);
+    if (!exempt.capturing()) return padded_spectrum(pl, pl->ctx->stream);
     hipStream_t aside = nullptr;
-    int st = ASARF_OK;
-    if (hipStreamCreateWithFlags(&aside, hipStreamNonBlocking) != hipSuccess) {
-        st = set_error(ASARF_EHIP, "asarf_plan: stream for the chirp spectrum");
-    } else {
-        st = padded_spectrum(pl, aside);
-        if (hipStreamSynchronize(aside) != hipSuccess && st == ASARF_OK)
-            st = set_error(ASARF_EHIP, "asarf_plan: chirp spectrum of %d samples", pl->nrp);
-        (void)hipStreamDestroy(aside);
-    }
-    HIP_CHECK(hipThreadExchangeStreamCaptureMode(&mode));
+    HIP_CHECK(hipStreamCreateWithFlags(&aside, hipStreamNonBlocking));
+    int st = padded_spectrum(pl, aside);
+    if (hipStreamSynchronize(aside) != hipSuccess && st == ASARF_OK)
+        st = set_error(ASARF_EHIP, "asarf_plan: chirp spectrum of %d samples", pl->nrp);
+    (void)hipStreamDestroy(aside);
     return st;
 }
 
