@@ -35,8 +35,9 @@ def test_short_first_pass(n1, cols, tmp_path):
 @pytest.mark.parametrize("n1,n2", [(n, 49) for n in (16, 18, 20, 21, 24, 25, 27, 28, 30)] +
                          [(98, n) for n in (16, 21, 25, 30)] + [(32, 35)])
 def test_register_lengths_in_both_passes(n1, n2, tmp_path):
-    """16 to 30 points in registers as the strided first pass and as the contiguous second one, and the first lengths
-    past them: against numpy in FP64 with the bound of test_short_first_pass (at most 2940 points)."""
+    """16 to 30 points as the strided first pass and as the contiguous second one, in launches too small for the register
+    kernel, and the first lengths past them: against numpy in FP64 with the bound of test_short_first_pass (at most 2940
+    points)."""
     ctx = focus.Context(0)
     path = str(tmp_path / "tune.txt")
     focus.tune_save(ctx, path)
@@ -54,14 +55,16 @@ def test_register_lengths_in_both_passes(n1, n2, tmp_path):
     ctx.close()
 
 
-@pytest.mark.parametrize("n1", [16, 18, 20, 21, 24, 25, 27, 28, 30])
-def test_register_kernel_takes_launches_that_fill_the_chip(n1, tmp_path):
-    """n1 x 49 on 2817 columns (12 x 49 workgroups: registers) and on the first 257 of them alone (2 x 49: LDS): both
-    within the bound of test_short_first_pass of numpy in FP64, and not the same sums in the same order."""
+@pytest.mark.parametrize("n1,n2", [(n, 49) for n in (16, 18, 20, 21, 24, 25, 27, 28, 30)] +
+                         [(98, n) for n in (16, 21, 25, 30)])
+def test_register_kernel_takes_launches_that_fill_the_chip(n1, n2, tmp_path):
+    """16 to 30 points as either pass on 2817 columns (12 workgroups for each of 49 or 98 groups: registers) and on the
+    first 257 of them alone (2 for each: LDS): both within the bound of test_short_first_pass of numpy in FP64, and not
+    the same sums in the same order."""
     ctx = focus.Context(0)
     path = str(tmp_path / "tune.txt")
     focus.tune_save(ctx, path)
-    n = n1 * 49
+    n = n1 * n2
     with open(path, "a") as f:
         f.write(f"col {n} {n1}\n")
     focus.tune_load(ctx, path)
